@@ -387,7 +387,9 @@ __global__ __launch_bounds__(64 * NW) void k_pairs(PairArgs<PREC> a) {
 // in the reference's orientation (lower index first), so both atoms see the
 // same value; the lower atom records the pair's energy and virial.  FP64
 // arithmetic in every form.  It reads only positions and charges, so it can
-// run beside the pair kernel.
+// run beside the pair kernel.  ENE false: forces only, no records (latency
+// of the block's seven sums: 12.6 -> 10.3 us on the 18.4k-atom slab, 5.1 ->
+// 3.9 us on 5k atoms of water).
 // k_combine: one thread per atom, the slot-order pair forces and the
 // atom-order accumulators (PME, bonded, excluded pairs) summed into the FP64
 // output and cleared for the next call.  No atomics.
@@ -402,7 +404,7 @@ struct CombineArgs {
   double *red;
 };
 
-template <class A, bool SPLIT>
+template <class A, bool SPLIT, bool ENE>
 __global__ __launch_bounds__(256) void k_excl(CombineArgs a, A *__restrict__ fat,
                                               A *__restrict__ fatc) {
   double ev[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -441,7 +443,7 @@ __global__ __launch_bounds__(256) void k_excl(CombineArgs a, A *__restrict__ fat
       if (SPLIT) acc_add(&fatc[3 * i + d], fe[d]);
     }
   }
-  block_record<7, 4>(ev, a.red + (size_t)blockIdx.x * PGK_REC);
+  if (ENE) block_record<7, 4>(ev, a.red + (size_t)blockIdx.x * PGK_REC);
 }
 
 template <class A, bool SPLIT>
@@ -588,7 +590,7 @@ static CombineArgs combine_args(pgk_ctx *c, bool do_pair) {
 }
 
 template <class A>
-static int launch_excl(pgk_ctx *c, bool split, int *off, int *nrec) {
+static int launch_excl(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
   CombineArgs a = combine_args(c, true);
   const int nblk = pgk_grid_blocks(c->natom, 256);
   *off = c->red_used;
@@ -596,10 +598,9 @@ static int launch_excl(pgk_ctx *c, bool split, int *off, int *nrec) {
   a.red = c->d_red + (size_t)c->red_used * PGK_REC;
   c->red_used += nblk;
   A *fat = reinterpret_cast<A *>(c->d_fat), *fatc = reinterpret_cast<A *>(c->d_fat_c);
-  if (split)
-    k_excl<A, true><<<nblk, 256, 0, c->stream>>>(a, fat, fatc);
-  else
-    k_excl<A, false><<<nblk, 256, 0, c->stream>>>(a, fat, fatc);
+  auto kf = split ? k_excl<A, true, true>   // the per-class forces come with their energies
+                  : (ene ? k_excl<A, false, true> : k_excl<A, false, false>);
+  kf<<<nblk, 256, 0, c->stream>>>(a, fat, fatc);
   HIP_CHECK(hipGetLastError());
   return PGK_OK;
 }
@@ -607,13 +608,13 @@ static int launch_excl(pgk_ctx *c, bool split, int *off, int *nrec) {
 // The excluded-pair correction of the listed pair terms into the atom-order
 // accumulators, with its energy/virial records (*nrec = 0 when the system
 // has no exclusions).
-int pgk_excl_launch(pgk_ctx *c, bool split, int *off, int *nrec) {
+int pgk_excl_launch(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
   *nrec = 0;
   if (c->nexclpair <= 0) return PGK_OK;
   switch (c->precision) {
-    case PGK_PREC_FP64: return launch_excl<double>(c, split, off, nrec);
-    case PGK_PREC_MIXED: return launch_excl<unsigned long long>(c, split, off, nrec);
-    default: return launch_excl<float>(c, split, off, nrec);
+    case PGK_PREC_FP64: return launch_excl<double>(c, split, ene, off, nrec);
+    case PGK_PREC_MIXED: return launch_excl<unsigned long long>(c, split, ene, off, nrec);
+    default: return launch_excl<float>(c, split, ene, off, nrec);
   }
 }
 

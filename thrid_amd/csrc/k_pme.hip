@@ -1158,7 +1158,8 @@ struct ConvArgs {
 // returns eterm (0 outside |m| <= rkcut) and adds the mode's energy and
 // virial terms, weighted for the half spectrum, to ev.  mh2 = m2/L2 and s2
 // (+1 on the k2 Nyquist plane, else -1) belong to k2; b1 b2 b3 are the
-// B-spline moduli of h, k2, k3.
+// B-spline moduli of h, k2, k3.  ENE false: eterm only.
+template <bool ENE>
 __device__ __forceinline__ double conv_mode(const ConvArgs &ca, int h, int k3, double mh2,
                                             double s2, double b1, double b2, double b3,
                                             double zx, double zy, double (&ev)[8]) {
@@ -1175,6 +1176,7 @@ __device__ __forceinline__ double conv_mode(const ConvArgs &ca, int h, int k3, d
     const double denom = ca.pivol * b1 * b2 * b3 * msq;
     const double ex = exp(-ca.fac * msq);
     eterm = ex / denom;
+    if (!ENE) return eterm;
     const double vterm = 2.0 * (ca.fac * msq + 1.0) / msq;
     const double struc2 = zx * zx + zy * zy;
     const bool single = (h == 0) || ((K1 & 1) == 0 && h == K1 / 2);
@@ -1204,6 +1206,8 @@ __device__ __forceinline__ double conv_mode(const ConvArgs &ca, int h, int k3, d
 // exp(-fac mh_d^2) and the moduli as reciprocals, so that a mode costs one
 // division.  e12 = exp(-fac (mh1^2 + mh2^2)) as a product, r12 = 1/(pi V b1 b2),
 // e3 = exp(-fac mh3^2), r3 = 1/b3; the cutoff test is the reference's.
+// ENE false: eterm only.
+template <bool ENE>
 __device__ __forceinline__ double conv_mode_f(const ConvArgs &ca, int h, int k3, double mh1,
                                               double mh2, double s2, double e12, double r12,
                                               double e3, double r3, double zx, double zy,
@@ -1218,6 +1222,7 @@ __device__ __forceinline__ double conv_mode_f(const ConvArgs &ca, int h, int k3,
     const double rm = 1.0 / msq;
     const double ex = e12 * e3;
     eterm = ex * (r12 * r3) * rm;
+    if (!ENE) return eterm;
     const double vterm = 2.0 * (ca.fac * msq + 1.0) * rm;
     const double struc2 = zx * zx + zy * zy;
     const bool single = (h == 0) || ((K1 & 1) == 0 && h == K1 / 2);
@@ -1244,8 +1249,12 @@ __device__ __forceinline__ double conv_mode_f(const ConvArgs &ca, int h, int k3,
 }
 
 // z pass with the register FFT and the convolution between the forward and
-// the backward transform; LPW lines per wavefront, h fastest across lines
-template <int PREC, class F>
+// the backward transform; LPW lines per wavefront, h fastest across lines.
+// ENE false (an MD step whose energies nobody reads): the energy and virial
+// terms, three quarters of the FP64 work of a mode, and their record are left
+// out (64 x 64 x 192 mixed 29.9 -> 26.0 us, 40^3 mixed 11.5 -> 9.0 us; at
+// 128^3 the pass waits for memory, 26 us beside the pair kernel either way).
+template <int PREC, class F, bool ENE>
 __global__ __launch_bounds__(64) void k_fft_z_conv_reg(void *cgrid, const void *twv, ConvArgs ca,
                                                        double *red) {
   using R = typename Prec<PREC>::real;
@@ -1293,8 +1302,8 @@ __global__ __launch_bounds__(64) void k_fft_z_conv_reg(void *cgrid, const void *
       const int k3 = t + F::N2 * q + F::N1 * kk;
       C &z = x[q * F::N2 + kk];
       if (valid && !(h == 0 && k2 == 0 && k3 == 0)) {   // m = 0 left untouched
-        const double eterm = conv_mode_f(ca, h, k3, mh1, mh2, s2, e12, r12, se3[k3], sr3[k3],
-                                         (double)z.x, (double)z.y, ev);
+        const double eterm = conv_mode_f<ENE>(ca, h, k3, mh1, mh2, s2, e12, r12, se3[k3],
+                                              sr3[k3], (double)z.x, (double)z.y, ev);
         z.x = (R)(eterm * (double)z.x);
         z.y = (R)(eterm * (double)z.y);
       }
@@ -1313,12 +1322,12 @@ __global__ __launch_bounds__(64) void k_fft_z_conv_reg(void *cgrid, const void *
       for (int kk = 0; kk < F::N2; kk++)
         cg[base + (size_t)(t + F::N2 * q + F::N1 * kk) * zstride] = x[q * F::N2 + kk];
   }
-  block_record<8, 1>(ev, red + (size_t)blockIdx.x * PGK_REC);
+  if (ENE) block_record<8, 1>(ev, red + (size_t)blockIdx.x * PGK_REC);
 }
 
 // z pass with the influence-function convolution between the forward and the
-// backward transform (scalar_sum, fft_pme.F90:544-690)
-template <int PREC>
+// backward transform (scalar_sum, fft_pme.F90:544-690); ENE as above
+template <int PREC, bool ENE>
 __global__ __launch_bounds__(256) void k_fft_z_conv(void *cgrid, int TW, FftPlan p,
                                                      const void *twv, ConvArgs ca,
                                                      double *red) {
@@ -1372,8 +1381,8 @@ __global__ __launch_bounds__(256) void k_fft_z_conv(void *cgrid, int TW, FftPlan
     if (h >= H) continue;
     if (h == 0 && k2 == 0 && k3 == 0) continue;   // m = 0 left untouched
     C z = pa[l * ls + k3];
-    const double eterm = conv_mode(ca, h, k3, mh2, s2, sb1[l], bsp2, sb3[k3], (double)z.x,
-                                   (double)z.y, ev);
+    const double eterm = conv_mode<ENE>(ca, h, k3, mh2, s2, sb1[l], bsp2, sb3[k3], (double)z.x,
+                                        (double)z.y, ev);
     z.x = (R)(eterm * (double)z.x);
     z.y = (R)(eterm * (double)z.y);
     pa[l * ls + k3] = z;
@@ -1384,7 +1393,7 @@ __global__ __launch_bounds__(256) void k_fft_z_conv(void *cgrid, int TW, FftPlan
     int k3 = t >> lt, l = t & (TW - 1);
     if (h0 + l < H) cg[(size_t)k3 * zstride + (size_t)(h0 + l) * K2 + k2] = pa[l * ls + k3];
   }
-  block_record<8, 4>(ev, red + (size_t)blockIdx.x * PGK_REC);
+  if (ENE) block_record<8, 4>(ev, red + (size_t)blockIdx.x * PGK_REC);
 }
 
 // Per-atom reciprocal virial, component comp (0..5: xx yy zz xy xz yz) of
@@ -1448,7 +1457,8 @@ __global__ __launch_bounds__(256) void k_fft_z_vir(void *cgrid, int TW, FftPlan 
     double g = 0.0;
     if (h != 0 || k2 != 0 || k3 != 0) {
       double ev[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      const double eterm = conv_mode(ca, h, k3, mh2, s2, sb1[l], bsp2, sb3[k3], 0.0, 0.0, ev);
+      const double eterm =
+          conv_mode<false>(ca, h, k3, mh2, s2, sb1[l], bsp2, sb3[k3], 0.0, 0.0, ev);
       if (eterm != 0.0) {
         const int m1 = (h < nf1) ? h : h - K1;
         const int m3 = (k3 < nf3) ? k3 : k3 - K3;
@@ -1635,7 +1645,7 @@ int launch_prep(pgk_ctx *c) {
 }
 
 template <int PREC>
-int launch_pme(pgk_ctx *c, bool split, int *off, int *nrec) {
+int launch_pme(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
   using R = typename Prec<PREC>::real;
   using C = typename C2T<R>::type;
   using A = typename Prec<PREC>::acc;
@@ -1740,14 +1750,16 @@ int launch_pme(pgk_ctx *c, bool split, int *off, int *nrec) {
     using F = decltype(f);
     const int nb = (H * K2 + F::LPW - 1) / F::LPW;
     *nrec = nb;
-    k_fft_z_conv_reg<PREC, F><<<nb, 64, 0, st>>>(c->d_cgrid, tw3, ca, red);
+    if (ene) k_fft_z_conv_reg<PREC, F, true><<<nb, 64, 0, st>>>(c->d_cgrid, tw3, ca, red);
+    else k_fft_z_conv_reg<PREC, F, false><<<nb, 64, 0, st>>>(c->d_cgrid, tw3, ca, red);
   });
   if (!rz) {
     const int twz = lines_for(K3, csz, 16);
     const int bz = K2 * ((H + twz - 1) / twz);
     *nrec = bz;
-    k_fft_z_conv<PREC><<<bz, 256, fft_lds_bytes(twz, K3, csz) + (twz + K3) * sizeof(double),
-                         st>>>(c->d_cgrid, twz, p3, tw3, ca, red);
+    auto kf = ene ? k_fft_z_conv<PREC, true> : k_fft_z_conv<PREC, false>;
+    kf<<<bz, 256, fft_lds_bytes(twz, K3, csz) + (twz + K3) * sizeof(double), st>>>(
+        c->d_cgrid, twz, p3, tw3, ca, red);
   }
   c->red_used += *nrec;
   HIP_CHECK(hipGetLastError());
@@ -1847,11 +1859,11 @@ int pgk_pme_prepare(pgk_ctx *c) {
   return PGK_OK;
 }
 
-int pgk_pme_launch(pgk_ctx *c, bool split, int *off, int *nrec) {
+int pgk_pme_launch(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
   switch (c->precision) {
-    case PGK_PREC_FP64: return launch_pme<PGK_PREC_FP64>(c, split, off, nrec);
-    case PGK_PREC_MIXED: return launch_pme<PGK_PREC_MIXED>(c, split, off, nrec);
-    default: return launch_pme<PGK_PREC_FP32>(c, split, off, nrec);
+    case PGK_PREC_FP64: return launch_pme<PGK_PREC_FP64>(c, split, ene, off, nrec);
+    case PGK_PREC_MIXED: return launch_pme<PGK_PREC_MIXED>(c, split, ene, off, nrec);
+    default: return launch_pme<PGK_PREC_FP32>(c, split, ene, off, nrec);
   }
 }
 

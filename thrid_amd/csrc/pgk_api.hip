@@ -329,11 +329,11 @@ int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom
     HIP_CHECK(hipEventRecord(c->ev_fork, st));
     HIP_CHECK(hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
     c->stream = c->stream2;
-    rc = pgk_pme_launch(c, split, &seg_off[nseg], &seg_n[nseg]);
+    rc = pgk_pme_launch(c, split, energies, &seg_off[nseg], &seg_n[nseg]);
     if (!rc) {
       seg_kind[nseg++] = SEG_PME;
       if (!excl_main) {
-        rc = pgk_excl_launch(c, split, &seg_off[nseg], &seg_n[nseg]);
+        rc = pgk_excl_launch(c, split, energies, &seg_off[nseg], &seg_n[nseg]);
         if (!rc && seg_n[nseg] > 0) seg_kind[nseg++] = SEG_EXCL;
       }
     }
@@ -367,22 +367,23 @@ int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom
     seg_kind[nseg++] = SEG_PAIR;
   }
   if (do_ewk && !overlap) {
-    if ((rc = pgk_pme_launch(c, split, &seg_off[nseg], &seg_n[nseg]))) return rc;
+    if ((rc = pgk_pme_launch(c, split, energies, &seg_off[nseg], &seg_n[nseg]))) return rc;
     seg_kind[nseg++] = SEG_PME;
     c->pme_grid_ready = true;
   }
   pgk_prof_begin(c, PGK_PROF_BONDED);
-  if ((rc = pgk_bonded_launch2(c, m, mts_flag, seg_off, seg_n, seg_kind, &nseg, hf))) return rc;
+  if ((rc = pgk_bonded_launch2(c, m, mts_flag, seg_off, seg_n, seg_kind, &nseg, hf, energies)))
+    return rc;
   pgk_prof_end(c, PGK_PROF_BONDED);
   if (overlap) {
     if (excl_main) {
-      if ((rc = pgk_excl_launch(c, split, &seg_off[nseg], &seg_n[nseg]))) return rc;
+      if ((rc = pgk_excl_launch(c, split, energies, &seg_off[nseg], &seg_n[nseg]))) return rc;
       if (seg_n[nseg] > 0) seg_kind[nseg++] = SEG_EXCL;
     }
     HIP_CHECK(hipStreamWaitEvent(st, c->ev_join, 0));
   } else if (do_pair) {
     pgk_prof_begin(c, PGK_PROF_EXCL);
-    if ((rc = pgk_excl_launch(c, split, &seg_off[nseg], &seg_n[nseg]))) return rc;
+    if ((rc = pgk_excl_launch(c, split, energies, &seg_off[nseg], &seg_n[nseg]))) return rc;
     pgk_prof_end(c, PGK_PROF_EXCL);
     if (seg_n[nseg] > 0) seg_kind[nseg++] = SEG_EXCL;
   }

@@ -368,12 +368,13 @@ int pgk_list_count_pairs(pgk_ctx *c);   // fills c->npairs (counted lazily)
 int pgk_pairs_launch(pgk_ctx *c, bool want_fsplit, bool energies, int *red_off, int *red_n);
 int pgk_combine_launch(pgk_ctx *c, bool do_pair, bool split, double *fout, double *fvc,
                        double *fvl);
-int pgk_excl_launch(pgk_ctx *c, bool split, int *off, int *nrec);
-int pgk_pme_launch(pgk_ctx *c, bool want_fsplit, int *red_off, int *red_n);
+// energies false: the records of energies and virials are left out
+int pgk_excl_launch(pgk_ctx *c, bool split, bool energies, int *off, int *nrec);
+int pgk_pme_launch(pgk_ctx *c, bool want_fsplit, bool energies, int *red_off, int *red_n);
 int pgk_pme_prepare(pgk_ctx *c);
 int pgk_pme_prep(pgk_ctx *c, bool pack);
 int pgk_bonded_launch2(pgk_ctx *c, const pgk_mts *m, int mts_flag, int *seg_off, int *seg_n,
-                       int *seg_kind, int *nseg, bool hf);
+                       int *seg_kind, int *nseg, bool hf, bool energies);
 int pgk_hf_launch_pairs(pgk_ctx *c, bool do_pairs);
 // regions the W-array pair pass holds per wave in LDS (volume / surface forms)
 #define PGK_HF_W_MAXREG 64
