@@ -924,7 +924,7 @@ int pgk_destroy(pgk_ctx *c) {
                   c->d_grid, c->d_pgrid, c->d_cgrid, c->d_tw, c->d_twf, c->d_theta, c->d_tile,
                   c->d_hf_z, c->d_hf_typ, c->d_hf_com, c->d_hf_pe, c->d_hf_w,
                   c->d_hf_pe_out, c->d_hf_w_out, c->d_md_gstart, c->d_md_cij, c->d_md_fail,
-                  c->d_md_small,
+                  c->d_md_small, c->d_md_tri,
                   c->d_md_d2, c->d_md_minv, c->d_md_vel, c->d_md_pos_old, c->d_md_free, c->d_md_ke,
                   c->d_md_kenhc,
                   c->d_md_nhc, c->d_lt_ustart, c->d_lt_uatom, c->d_lt_ucom, c->d_lt_reg,
@@ -1481,7 +1481,7 @@ int pgk_md_setup(pgk_ctx *c, const pgk_md_desc *md) {
   // b and c the others, so the order reads (a,b), (a,c), (b,c).  Swapping the
   // two atoms of a constraint changes no result (both vectors change sign).
   const int ng = md->ncons > 0 ? md->ngroup : 0;
-  std::vector<int32_t> small(std::max(ng, 1), 0);
+  std::vector<int32_t> small(std::max(ng, 1), 0), tri(4 * (size_t)std::max(ng, 1), 0);
   for (int g = 0; g < ng; g++) {
     if (gs[g + 1] - gs[g] != 3) continue;
     const int k0 = gs[g];
@@ -1499,12 +1499,14 @@ int pgk_md_setup(pgk_ctx *c, const pgk_md_desc *md) {
       cij[2 * (k0 + q) + 1] = lab[q][1];
     }
     small[g] = 1;
+    const int rec[4] = {a, b, cc, k0};
+    for (int q = 0; q < 4; q++) tri[4 * (size_t)g + q] = rec[q];
   }
   int rc = set_device_ctx(c);
   if (rc) return rc;
   if ((rc = upload(&c->d_md_minv, minv)) || (rc = upload(&c->d_md_gstart, gs)) ||
       (rc = upload(&c->d_md_cij, cij)) || (rc = upload(&c->d_md_d2, d2)) ||
-      (rc = upload(&c->d_md_small, small)))
+      (rc = upload(&c->d_md_small, small)) || (rc = upload(&c->d_md_tri, tri)))
     return rc;
   std::vector<double> zero((size_t)3 * n, 0.0);
   std::vector<int32_t> one(1, 0);

@@ -294,6 +294,7 @@ struct pgk_ctx {
   double md_dt = 1.0, md_tol = 1e-10;
   int32_t *d_md_gstart = nullptr, *d_md_cij = nullptr, *d_md_fail = nullptr;
   int32_t *d_md_small = nullptr;
+  int32_t *d_md_tri = nullptr;     // [4*ngroup] a triangle group's atoms and first constraint
   bool md_all_tri = false;         // every group a triangle: fused half-step kernels
   bool md_graphs = false;          // pgk_md_run: replay plain steps from a captured graph
   bool md_batch_graphs = false;    // pgk_md_run_batch: the same, per replica
