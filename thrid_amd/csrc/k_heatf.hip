@@ -223,29 +223,28 @@ __global__ __launch_bounds__(256) void k_heatf_final(HeatfArgs a, const double *
   }
 }
 
-// flux form: collision row (class, region) = the bonded terms' sums in jcol
-// (heat-flux accumulator type AH) plus, for the pair classes, the pair pass's
-// per-block records in block order (block (row, component) per launch block,
-// fixed-order tree).  direct (bulk, one region): the pair pass's transport
+// flux form, bulk mode: collision row (class, region) = the bonded terms' sums
+// in jcol (heat-flux accumulator type AH) plus, for the pair classes, the pair
+// pass's per-block records in block order (block (row, component) per launch
+// block, fixed-order tree).  direct (one region): the pair pass's transport
 // sums too, into the transport record slot after the atom chunks' (tslot),
 // zero for the other terms.
 template <class AH>
-__global__ __launch_bounds__(256) void k_heatf_collect(int nreg, int bulk, int nblk,
+__global__ __launch_bounds__(256) void k_heatf_collect(int nreg, int nblk,
                                                        const AH *__restrict__ jcol,
                                                        const double *__restrict__ jpart,
                                                        double *__restrict__ pcol, int direct,
                                                        double *__restrict__ tslot) {
   const int row = blockIdx.x / 3, c = blockIdx.x % 3;   // row = class * nreg + region
-  const int k = row / nreg, r = row % nreg;
+  const int k = row / nreg;
   const int q = k - PGK_HF_ELIN;
   const bool pair = q >= 0 && q < 4;
   double v[2] = {0.0, 0.0};
-  if (pair && (bulk || c == 2)) {
-    const int stride = bulk ? 24 : 4 * nreg;
-    const int off = bulk ? 3 * q + c : q * nreg + r;
+  if (pair) {
+    const int off = 3 * q + c;
     for (int b = threadIdx.x; b < nblk; b += 256) {
-      v[0] += jpart[(size_t)b * stride + off];
-      if (direct) v[1] += jpart[(size_t)b * stride + 12 + off];
+      v[0] += jpart[(size_t)b * 24 + off];
+      if (direct) v[1] += jpart[(size_t)b * 24 + 12 + off];
     }
   }
   __shared__ double rec[PGK_REC];
@@ -290,7 +289,7 @@ int launch_heatf(pgk_ctx *c, const HeatfArgs &a, double *ptr, double *pcol) {
   if (c->hfdev.flux) {
     const int direct = a.ntr_slot > a.nsplit_tr;   // one region: its slot after the chunks'
     k_heatf_collect<AH><<<PGK_NHF * a.nreg * 3, 256, 0, st>>>(
-        a.nreg, a.bulk, pgk_grid_blocks(pgk_pair_waves(c), 4),
+        a.nreg, pgk_grid_blocks(pgk_pair_waves(c), 4),
         reinterpret_cast<const AH *>(c->hfdev.jcol), c->hfdev.jpart, pcol, direct,
         ptr + (size_t)a.nsplit_tr * (kNterm * 3));
   } else {
@@ -381,6 +380,14 @@ int pgk_heatf_launch(pgk_ctx *c, const double *d_vel, const double *d_mass,
     k_molevel<<<pgk_grid_blocks(c->hj_nmol, 256), 256, 0, c->stream>>>(
         c->hj_nmol, c->d_hj_mol_start, c->d_hj_mol_atoms, d_mass, d_vel, c->d_hj_molevel);
     HIP_CHECK(hipGetLastError());
+  }
+  if (h.flux && h.mode != PGK_HF_BULK) {   // the volume mode's flux form: k_hf_vol.hip
+    HfBinArgs b;
+    b.vel = d_vel;
+    b.mass = d_mass;
+    b.molevel = c->d_hj_molevel;
+    b.vstrm = d_vstrm;
+    return pgk_hf_vol_bins_launch(c, b, out ? out : c->d_hj_out);
   }
   if (h.nreg > 1) {   // many regions: the centres once, not once per region
     if ((rc = grow_dev((void **)&c->d_hj_cz, &c->hj_cz_cap, sizeof(double) * n))) return rc;

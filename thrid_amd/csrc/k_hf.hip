@@ -1,6 +1,7 @@
-// k_hf.hip - fused heat-flux pass over the listed pairs (pgk_calforce_heatf
-// and the MD loop's samples), and the export of calforce_hf's per-atom arrays
-// (whose pair pass is k_hf_w.hip).
+// k_hf.hip - fused heat-flux pass over the listed pairs in the bulk mode
+// (pgk_calforce_heatf and the MD loop's samples; the volume mode's is
+// k_hf_vol.hip), and the export of calforce_hf's per-atom arrays (whose pair
+// pass is k_hf_w.hip).
 //
 // Restates the per-atom part of ewaldrp_hf (ewaldr_hf.F90:8-670) in the
 // default build: for every listed pair with r <= rrcut the bare Coulomb
@@ -37,17 +38,11 @@ struct HfPairArgs {
   double rrsq;   // largest r^2 with sqrt(r^2) <= rrcut: r2 <= rrsq decides r <= rrcut exactly
 };
 
-__device__ __forceinline__ double r2_exact(const double *r) {
-#pragma clang fp contract(off)
-  return r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-}
-
 // Flux form of the pass (pgk_calforce_heatf): the same pairs, energies and
 // per-atom energy sums, but the collision part of calheatf is summed on the
-// spot, s = fi . (v_i + v_j) times the region weights, instead of scattering
-// W arrays.  Bulk: 4 pair classes x 3 components per lane in registers.
-// Volume: a [4][nreg] slice of LDS per wave, added to with LDS atomics.  Each
-// block then adds its waves in order into jpart[block].
+// spot, s = fi . (v_i + v_j) times the centres' separation, instead of
+// scattering W arrays: 4 pair classes x 3 components per lane in registers.
+// Each block then adds its waves in order into jpart[block].
 constexpr int kPairCls0 = PGK_HF_ELIN;   // ELIN, LJIN, ELC, VDW are 4..7
 
 // what an interaction needs besides its class, energy and force coefficient
@@ -55,21 +50,19 @@ struct FluxPair {
   bool seg;          // the centres' segment counts (not two MOLE atoms of one molecule...)
   double rw;         // r . (v_i + v_j)
   double w[3];       // v_i + v_j
-  double rc[3];      // centre separation (minimum image in the bulk form)
-  double ciz, cjz, rz;
+  double rc[3];      // centre separation (minimum image)
 };
 
 // one interaction of pair class Q (0 ELIN, 1 LJIN, 2 ELC, 3 VDW) with energy
 // e and force coefficient f (force on i = f r): half the energy to each
-// atom, and f (r . (v_i + v_j)) / 2 times the region weights to the flux.
-// DT (bulk form over the whole box, atom centres, transport velocities =
+// atom, and f (r . (v_i + v_j)) / 2 times the separation to the flux.
+// DT (one region over the whole box, atom centres, transport velocities =
 // the pair's velocities): the energies' share of the transport part,
 // e/2 (v_i + v_j), is summed here (tr) instead of per atom.
-template <int Q, bool BULK, bool DT>
+template <int Q, bool DT>
 __device__ __forceinline__ void flux_add(const FluxPair &fp, double e, double f,
                                          double (&ei)[4], double (&ej)[4],
-                                         double (&acc)[4][3], double (&tr)[4][3],
-                                         double &sv_out) {
+                                         double (&acc)[4][3], double (&tr)[4][3]) {
   if (DT) {
     const double he = 0.5 * e;
 #pragma unroll
@@ -80,110 +73,18 @@ __device__ __forceinline__ void flux_add(const FluxPair &fp, double e, double f,
   }
   if (!fp.seg) return;
   const double sv = f * fp.rw * 0.5;
-  if (BULK) {
 #pragma unroll
-    for (int n = 0; n < 3; n++) acc[Q][n] += fp.rc[n] * sv;
-  } else {
-    sv_out = sv;   // the region walk adds it once per pair, for both classes
-  }
-}
-
-// volume form: the pair's Coulomb (class qc) and LJ (class ql) shares times
-// the weight of every region its centres' segment crosses (zr: the regions'
-// bounds, z1 then z2, staged in LDS)
-__device__ __forceinline__ void flux_regions(const HfDev &h, const FluxPair &fp, int qc,
-                                             double svc, int ql, double svl, double *sl,
-                                             const double *zr) {
-  if (!fp.seg || (svc == 0.0 && svl == 0.0)) return;
-  const double lo = fmin(fp.ciz, fp.cjz), hi = fmax(fp.ciz, fp.cjz);
-  if (h.tiled) {
-    // ka, kb: the last region with z1 <= lo, hi (-1: none).  Regions below
-    // ka - 1 end below lo, regions above kb start above hi: the weight
-    // misses them.  ka - 1 ends at z1[ka]: it is weighed only when that is
-    // lo itself.  Regions strictly between ka and kb have lo < z1 < z2 <= hi,
-    // so both planes are crossed (or the upper plane holds the upper centre)
-    // and the weight is their signed width, as hf_volume_weight_z gives it.
-    const int nreg = h.nreg;
-    int ka = min(nreg - 1, max(-1, (int)floor((lo - h.ubz0) * h.ubwi)));
-    while (ka + 1 < nreg && zr[ka + 1] <= lo) ka++;
-    while (ka >= 0 && zr[ka] > lo) ka--;
-    int kb = min(nreg - 1, max(ka, (int)floor((hi - h.ubz0) * h.ubwi)));
-    while (kb + 1 < nreg && zr[kb + 1] <= hi) kb++;
-    while (kb > ka && zr[kb] > hi) kb--;
-    auto exact = [&](int ir) {
-      const double z1 = zr[ir], z2 = zr[nreg + ir];
-      if (hi < z1 || lo > z2) return;
-      const double ff = hf_volume_weight_z(z1, z2, fp.ciz, fp.cjz, fp.rc[2], fp.rz, 1.0);
-      if (ff == 0.0) return;
-      if (svc != 0.0) atomicAdd(&sl[qc * nreg + ir], ff * svc);
-      if (svl != 0.0) atomicAdd(&sl[ql * nreg + ir], ff * svl);
-    };
-    if (ka >= 1 && zr[ka] == lo) exact(ka - 1);
-    if (ka >= 0) exact(ka);
-    const bool neg = !(fp.rc[2] >= 0.0);
-    for (int ir = max(ka + 1, 0); ir < kb; ir++) {
-      const double wd = zr[nreg + ir] - zr[ir];
-      const double ff = neg ? -wd : wd;
-      if (svc != 0.0) atomicAdd(&sl[qc * nreg + ir], ff * svc);
-      if (svl != 0.0) atomicAdd(&sl[ql * nreg + ir], ff * svl);
-    }
-    if (kb > ka) exact(kb);
-    return;
-  }
-  int r0, r1;
-  hf_region_window(h, lo, hi, r0, r1);
-  for (int ir = r0; ir <= r1; ir++) {
-    const double z1 = zr[ir], z2 = zr[h.nreg + ir];
-    if (hi < z1 || lo > z2) continue;   // the segment misses the region
-    const double ff = hf_volume_weight_z(z1, z2, fp.ciz, fp.cjz, fp.rc[2], fp.rz, 1.0);
-    if (ff == 0.0) continue;
-    if (svc != 0.0) atomicAdd(&sl[qc * h.nreg + ir], ff * svc);
-    if (svl != 0.0) atomicAdd(&sl[ql * h.nreg + ir], ff * svl);
-  }
-}
-
-// Cross-lane exchange inside aligned groups of 8 lanes (DPP, no LDS):
-// quad_perm [1,0,3,2] = 0xB1, quad_perm [2,3,0,1] = 0x4E, row_half_mirror
-// (lane k <-> 7 - k) = 0x141.
-template <int CTRL>
-__device__ __forceinline__ double dpp8d(double v) {
-  int lo = __double2loint(v), hi = __double2hiint(v);
-  lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, false);
-  hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-// e[0..3] summed over each aligned group of 8 lanes (k = lane & 7) in four
-// exchanges: afterwards lanes k and k^1 hold the sum of e[k >> 1].  Step 1
-// pairs k with 7 - k (the low half keeps e0 and e1, the high half e2 and
-// e3), step 2 pairs k with k^2 (k & 2 keeps the second of its two), step 3
-// k with k^1.  The group's whole wave must be active.
-__device__ __forceinline__ double sum4x8(const double (&e)[4], int k) {
-  const bool hi = (k & 4) != 0;
-  const double a0 = (hi ? e[2] : e[0]) + dpp8d<0x141>(hi ? e[0] : e[2]);
-  const double a1 = (hi ? e[3] : e[1]) + dpp8d<0x141>(hi ? e[1] : e[3]);
-  const bool b1 = (k & 2) != 0;
-  const double b = (b1 ? a1 : a0) + dpp8d<0x4E>(b1 ? a0 : a1);
-  return b + dpp8d<0xB1>(b);
-}
-
-// 1/sqrt(r^2) in the compute type: FP64 divide of the root, or FP32's
-// hardware reciprocal root (about one ulp)
-template <class R> __device__ __forceinline__ R hf_rinv(double r2);
-template <> __device__ __forceinline__ double hf_rinv<double>(double r2) { return 1.0 / sqrt(r2); }
-template <> __device__ __forceinline__ float hf_rinv<float>(double r2) {
-  return __builtin_amdgcn_rsqf((float)r2);
+  for (int n = 0; n < 3; n++) acc[Q][n] += fp.rc[n] * sv;
 }
 
 // CH: the chunked form, one wave per work item (64 list entries of one
 // cluster) instead of one wave per cluster; the i atom's energies are then
 // added once per item
-template <class AH, bool BULK, bool CH, bool DT>
+template <class AH, bool CH, bool DT>
 __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
   // the mixed form (fixed-point accumulators) computes the pair terms in FP32
   using R = typename std::conditional<std::is_same<AH, unsigned long long>::value, float,
                                       double>::type;
-  extern __shared__ double lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int ci = blockIdx.x * 4 + wave, chunk = 0;
   if (CH) {
@@ -195,18 +96,7 @@ __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
       chunk = item & 31;
     }
   }
-  const int nreg = h.nreg;
   double acc[4][3] = {}, tr[4][3] = {};
-  double *sl = lds + (size_t)wave * 4 * nreg;   // volume: this wave's slice
-  double *zr = lds + (size_t)16 * nreg;           // volume: the regions' bounds
-  if (!BULK) {
-    for (int k = lane; k < 4 * nreg; k += 64) sl[k] = 0.0;
-    for (int k = threadIdx.x; k < nreg; k += 256) {
-      zr[k] = h.z1[k];
-      zr[nreg + k] = h.z2[k];
-    }
-    __syncthreads();
-  }
   if (ci < p.ncl) {
     const int ii = lane & 7, jq = (lane >> 3) & 3, hs = lane >> 5;
     // the i atom's slot, loaded once for the whole list (padding slots, ai =
@@ -235,7 +125,7 @@ __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
         const double4 xj = p.xq[js];
         double r[3] = {xi.x - xj.x, xi.y - xj.y, xi.z - xj.z};
         for (int d = 0; d < 3; d++) r[d] = r[d] - h.L[d] * rint(r[d] * h.Li[d]);
-        const double r2 = r2_exact(r);
+        const double r2 = hf_r2_exact(r);
         if (r2 <= p.sqcut) {
           // the cutoff tests stay exact FP64 decisions; the pair terms are in
           // the compute type R (FP32 in the mixed form: one hardware rsqrt)
@@ -243,37 +133,31 @@ __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
           const R rinv2 = rinv1 * rinv1;
           const bool same = moli == p.mol[js];
           const double4 ccj = p.cen[js];
-          // the centres' separation and, in the volume form, whether it counts
-          double rc[3], rz = 0.0;
+          // the centres' separation and whether it counts
+          double rc[3];
           bool seg = true;
-          if (BULK && cci.w != 0.0 && ccj.w != 0.0) {
-            // two atom centres in the bulk form: the centres' minimum image
-            // is the pair's own r (round and rint differ only at a
-            // half-box tie, which no listed pair reaches)
+          if (cci.w != 0.0 && ccj.w != 0.0) {
+            // two atom centres: the centres' minimum image is the pair's own
+            // r (round and rint differ only at a half-box tie, which no
+            // listed pair reaches)
             for (int d = 0; d < 3; d++) rc[d] = r[d];
           } else {
             seg = !(cci.w == 0.0 && ccj.w == 0.0 && same);
             rc[0] = cci.x - ccj.x;
             rc[1] = cci.y - ccj.y;
             rc[2] = cci.z - ccj.z;
-            if (BULK) {
-              for (int d = 0; d < 3; d++) rc[d] = rc[d] - h.L[d] * round(rc[d] * h.Li[d]);
-            } else {
-              rz = fabs(rc[2]);
-              seg = seg && rz * h.Li[2] < 0.5;
-            }
+            for (int d = 0; d < 3; d++) rc[d] = rc[d] - h.L[d] * round(rc[d] * h.Li[d]);
           }
           // s = fi . v_i - fj . v_j with fj = -fi, per unit force coefficient
           const double4 vj = p.v4[js];
           const double w[3] = {vi.x + vj.x, vi.y + vj.y, vi.z + vj.z};
           const double rw = r[0] * w[0] + r[1] * w[1] + r[2] * w[2];
-          const FluxPair fp{seg, rw, {w[0], w[1], w[2]}, {rc[0], rc[1], rc[2]}, cci.z, ccj.z, rz};
-          double svc = 0.0, svl = 0.0;
+          const FluxPair fp{seg, rw, {w[0], w[1], w[2]}, {rc[0], rc[1], rc[2]}};
           if (r2 <= p.rrsq) {
             const R qq = (R)xi.w * (R)xj.w;
             const R ph = qq * rinv1;
-            if (same) flux_add<0, BULK, DT>(fp, ph, ph * rinv2, ei, ej, acc, tr, svc);
-            else flux_add<2, BULK, DT>(fp, ph, ph * rinv2, ei, ej, acc, tr, svc);
+            if (same) flux_add<0, DT>(fp, ph, ph * rinv2, ei, ej, acc, tr);
+            else flux_add<2, DT>(fp, ph, ph * rinv2, ei, ej, acc, tr);
           }
           if (r2 <= p.sqcut2) {
             const int tp = typi + p.ntype * p.ct[js];
@@ -284,17 +168,16 @@ __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
               const R t12 = t6 * t6;
               const R pot = ep * (t12 - (R)2 * t6);
               const R ft = (R)12 * ep * (t12 - t6) * rinv2;
-              if (same) flux_add<1, BULK, DT>(fp, pot, ft, ei, ej, acc, tr, svl);
-              else flux_add<3, BULK, DT>(fp, pot, ft, ei, ej, acc, tr, svl);
+              if (same) flux_add<1, DT>(fp, pot, ft, ei, ej, acc, tr);
+              else flux_add<3, DT>(fp, pot, ft, ei, ej, acc, tr);
             }
           }
-          if (!BULK) flux_regions(h, fp, same ? 0 : 2, svc, same ? 1 : 3, svl, sl, zr);
         }
       }
       if (!DT) {
         // the j atom's four class energies summed over its 8 lanes; lanes
         // ii and ii^1 then hold class (ii >> 1) and one of them adds it
-        const double sj4 = sum4x8(ej, ii);
+        const double sj4 = hf_sum4x8(ej, ii);
         if (aj >= 0 && (ii & 1) == 0 && sj4 != 0.0)
           hf_pe_add<AH>(h, kPairCls0 + (ii >> 1), aj, sj4);
       }
@@ -305,32 +188,24 @@ __global__ __launch_bounds__(256) void k_hf_pairs_flux(HfPairArgs p, HfDev h) {
         if (ei[q] != 0.0) hf_pe_add<AH>(h, kPairCls0 + q, ai, ei[q]);
     }
   }
-  if (BULK) {
-    // per block: the 12 flux sums, then (DT) the 12 transport sums, else 0
-    __shared__ double wsum[4][24];
+  // per block: the 12 flux sums, then (DT) the 12 transport sums, else 0
+  __shared__ double wsum[4][24];
 #pragma unroll
-    for (int q = 0; q < 4; q++)
+  for (int q = 0; q < 4; q++)
 #pragma unroll
-      for (int n = 0; n < 3; n++) {
-        const double t = wave_sum(acc[q][n]);
-        const double u = DT ? wave_sum(tr[q][n]) : 0.0;
-        if (lane == 0) {
-          wsum[wave][3 * q + n] = t;
-          wsum[wave][12 + 3 * q + n] = u;
-        }
+    for (int n = 0; n < 3; n++) {
+      const double t = wave_sum(acc[q][n]);
+      const double u = DT ? wave_sum(tr[q][n]) : 0.0;
+      if (lane == 0) {
+        wsum[wave][3 * q + n] = t;
+        wsum[wave][12 + 3 * q + n] = u;
       }
-    __syncthreads();
-    if (threadIdx.x < 24)
-      h.jpart[(size_t)blockIdx.x * 24 + threadIdx.x] =
-          ((wsum[0][threadIdx.x] + wsum[1][threadIdx.x]) + wsum[2][threadIdx.x]) +
-          wsum[3][threadIdx.x];
-  } else {
-    __syncthreads();
-    const int nv = 4 * nreg;
-    for (int k = threadIdx.x; k < nv; k += 256)
-      h.jpart[(size_t)blockIdx.x * nv + k] =
-          ((lds[k] + lds[nv + k]) + lds[2 * nv + k]) + lds[3 * nv + k];
-  }
+    }
+  __syncthreads();
+  if (threadIdx.x < 24)
+    h.jpart[(size_t)blockIdx.x * 24 + threadIdx.x] =
+        ((wsum[0][threadIdx.x] + wsum[1][threadIdx.x]) + wsum[2][threadIdx.x]) +
+        wsum[3][threadIdx.x];
 }
 
 // accumulators -> doubles in the caller's layout: pot_atm[class][atom] and the
@@ -382,6 +257,7 @@ int launch_hf(pgk_ctx *c, bool do_pairs) {
     const int nblk = pgk_grid_blocks(pgk_pair_waves(c), 4);
     const bool ch = pgk_pair_chunked(c);
     if (!h.flux) return pgk_hf_w_launch(c);   // per-atom arrays: k_hf_w.hip
+    if (h.mode != PGK_HF_BULK) return pgk_hf_vol_launch(c);
     // the flux form reads its atoms' data per cluster slot
     const int nslot = c->ncl * PGK_CL;
     int rc;
@@ -401,22 +277,11 @@ int launch_hf(pgk_ctx *c, bool do_pairs) {
     p.ct = c->d_ct;
     p.lj = c->d_ljp64;
     // the pair energies' transport share summed in the pass (see flux_add)
-    const bool dt = h.mode == PGK_HF_BULK && h.direct_ok && h.vel == h.tvel;
+    const bool dt = h.direct_ok && h.vel == h.tvel;
     c->hfdev.direct_tr = dt ? 1 : 0;
-    if (h.mode == PGK_HF_BULK) {
-      auto kf = ch ? (dt ? k_hf_pairs_flux<AH, true, true, true>
-                         : k_hf_pairs_flux<AH, true, true, false>)
-                   : (dt ? k_hf_pairs_flux<AH, true, false, true>
-                         : k_hf_pairs_flux<AH, true, false, false>);
-      kf<<<nblk, 256, 0, st>>>(p, h);
-    } else {
-      const size_t lds = sizeof(double) * 18 * (size_t)h.nreg;   // 4 wave slices + bounds
-      auto kf = ch ? k_hf_pairs_flux<AH, false, true, false>
-                   : k_hf_pairs_flux<AH, false, false, false>;
-      const int lr = pgk_lds_limit((const void *)kf, lds);
-      if (lr) return lr;
-      kf<<<nblk, 256, lds, st>>>(p, h);
-    }
+    auto kf = ch ? (dt ? k_hf_pairs_flux<AH, true, true> : k_hf_pairs_flux<AH, true, false>)
+                 : (dt ? k_hf_pairs_flux<AH, false, true> : k_hf_pairs_flux<AH, false, false>);
+    kf<<<nblk, 256, 0, st>>>(p, h);
     HIP_CHECK(hipGetLastError());
   }
   return PGK_OK;

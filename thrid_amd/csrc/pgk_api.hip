@@ -930,7 +930,7 @@ int pgk_destroy(pgk_ctx *c) {
                   c->d_md_nhc, c->d_lt_ustart, c->d_lt_uatom, c->d_lt_ucom, c->d_lt_reg,
                   c->d_lt_cnt, c->d_lt_mass, c->d_lt_frand, c->d_lt_det, c->d_lt_sreg, c->d_md_vstrm,
                   c->d_hf_vstrm, c->d_hj_vpec, c->d_vgrid,
-                  c->d_vir6, c->d_hfw_xq, c->d_hfw_cen, c->d_hfw_mol, c->d_hfw_v, c->d_tl_start,
+                  c->d_vir6, c->d_hfv_mt, c->d_hfv_acc, c->d_hfw_xq, c->d_hfw_cen, c->d_hfw_mol, c->d_hfw_v, c->d_tl_start,
                   c->d_tl_src, c->d_tl_mask, c->d_hj_vel, c->d_hj_mass, c->d_hj_molevel,
                   c->d_hj_cz,
                   c->d_hj_part, c->d_hj_out, c->d_hj_mol_start, c->d_hj_mol_atoms,
@@ -1238,19 +1238,23 @@ static int hf_setup(pgk_ctx *c, const pgk_hf_desc *hf, bool flux, const char *wh
                     ? 1
                     : 0;
   h.direct_tr = 0;
+  h.vol_pairs = 0;
   h.jcol = nullptr;
   h.jpart = nullptr;
   if (flux) {
     const size_t jcol_b = sizeof(double) * PGK_NHF * (size_t)nreg * 3;
     const size_t nblk = (size_t)pgk_grid_blocks(std::max<int64_t>(pgk_pair_waves(c), 1), 4);
-    // bulk: 12 flux sums and 12 transport sums per block; volume: [4][nreg]
-    const size_t jpart_b =
-        sizeof(double) * nblk * (hf->mode == PGK_HF_BULK ? 24 : 4 * (size_t)nreg);
+    // bulk: 12 flux sums and 12 transport sums per block; volume: 4 classes of
+    // two words per region (k_hf_vol.hip)
+    const bool bulk = hf->mode == PGK_HF_BULK;
+    const size_t jpart_b = sizeof(double) * (bulk ? nblk * 24 : 8 * (size_t)nreg);
     if ((rc = grow_dev((void **)&c->d_hj_jcol, &c->hj_jcol_cap, jcol_b)) ||
         (rc = grow_dev((void **)&c->d_hj_jpart, &c->hj_jpart_cap, jpart_b)))
       return rc;
-    // the per-atom energies and both flux sums start at zero: one launch
-    if ((rc = pgk_zero3_launch(st, c->d_hf_pe, pe_b / 8, c->d_hj_jcol, jcol_b / 8, c->d_hj_jpart,
+    // the per-atom energies (volume mode: bonded terms only) and the flux sums
+    // start at zero: one launch
+    const size_t pe0 = bulk || pgk_has_bonded(c) ? pe_b / 8 : 0;
+    if ((rc = pgk_zero3_launch(st, c->d_hf_pe, pe0, c->d_hj_jcol, jcol_b / 8, c->d_hj_jpart,
                                jpart_b / 8)))
       return rc;
     h.jcol = c->d_hj_jcol;

@@ -275,3 +275,60 @@ __device__ void calvirihf_dev(const HfDev &h, int i, int j, const double *fi, co
     }
   }
 }
+
+// |r|^2 without contraction: the reference's cutoff decision
+__device__ __forceinline__ double hf_r2_exact(const double *r) {
+#pragma clang fp contract(off)
+  return r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+}
+
+// Cross-lane exchange inside aligned groups of 8 lanes (DPP, no LDS):
+// quad_perm [1,0,3,2] = 0xB1, quad_perm [2,3,0,1] = 0x4E, row_half_mirror
+// (lane k <-> 7 - k) = 0x141.
+template <int CTRL>
+__device__ __forceinline__ double dpp8d(double v) {
+  int lo = __double2loint(v), hi = __double2hiint(v);
+  lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, false);
+  hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+
+// e[0..3] summed over each aligned group of 8 lanes (k = lane & 7) in four
+// exchanges: afterwards lanes k and k^1 hold the sum of e[k >> 1].  Step 1
+// pairs k with 7 - k (the low half keeps e0 and e1, the high half e2 and
+// e3), step 2 pairs k with k^2 (k & 2 keeps the second of its two), step 3
+// k with k^1.  The group's whole wave must be active.
+__device__ __forceinline__ double hf_sum4x8(const double (&e)[4], int k) {
+  const bool hi = (k & 4) != 0;
+  const double a0 = (hi ? e[2] : e[0]) + dpp8d<0x141>(hi ? e[0] : e[2]);
+  const double a1 = (hi ? e[3] : e[1]) + dpp8d<0x141>(hi ? e[1] : e[3]);
+  const bool b1 = (k & 2) != 0;
+  const double b = (b1 ? a1 : a0) + dpp8d<0x4E>(b1 ? a0 : a1);
+  return b + dpp8d<0xB1>(b);
+}
+
+// 1/sqrt(r^2) in the compute type: FP64 divide of the root, or FP32's
+// hardware reciprocal root (about one ulp)
+template <class R> __device__ __forceinline__ R hf_rinv(double r2);
+template <> __device__ __forceinline__ double hf_rinv<double>(double r2) { return 1.0 / sqrt(r2); }
+template <> __device__ __forceinline__ float hf_rinv<float>(double r2) {
+  return __builtin_amdgcn_rsqf((float)r2);
+}
+
+// ---- the volume mode's flux form (k_hf_vol.hip) -----------------------------
+// what the regions' sums read: the items (list slots with the pair pass's
+// sums, or atoms), their centres, velocities and energies
+struct HfBinArgs {
+  int natom, nitem, nreg, nsplit, per, tiled;   // per: items of a part
+  double ubz0, ubwi;
+  double Lx, Ly, Lz;
+  const double *z1, *z2;
+  const int32_t *order;          // item -> atom (-1: padding), or null: identity
+  const int32_t *hftyp, *molid;
+  const double *molecom, *pos, *vel, *mass, *molevel;
+  const double *vstrm;           // streaming velocities for the kinetic energies, or null
+  const void *pe;                // bonded energies [class][atom], or null: no bonded terms
+  const void *acc;               // the pair pass's sums per slot, or null
+};
+int pgk_hf_vol_launch(pgk_ctx *c);
+int pgk_hf_vol_bins_launch(pgk_ctx *c, HfBinArgs a, double *out);

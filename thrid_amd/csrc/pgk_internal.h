@@ -60,7 +60,7 @@ void pgk_set_error(const std::string &msg);
 // eref / (amu A^2 fs^-2): a = F/m * PGK_MD_CONV, KE = m v^2 / 2 / PGK_MD_CONV
 #define PGK_MD_CONV (6.9511042e-21 / 1.66053907e-17)
 
-// volume regions of the flux form: the pair pass keeps [4][nreg] doubles of
+// volume regions of the flux form: the regions' sums keep [17][nreg] doubles of
 // LDS per wave
 #define PGK_HEATF_MAXREG 1024
 
@@ -94,8 +94,10 @@ struct HfDev {
   // energies' transport share itself (direct_tr) instead of per-atom energies
   const double *tvel = nullptr;
   int direct_ok = 0, direct_tr = 0;
+  int vol_pairs = 0;                           // volume mode: the pair pass has run
   double *jcol = nullptr;   // [PGK_NHF][nreg][3] sums, heat-flux accumulator type (int64 fixed point in the mixed form)
-  double *jpart = nullptr;                     // pair pass: per-block records
+  // bulk pair pass: per-block records; volume: sums of the pairs on a plane
+  double *jpart = nullptr;
 };
 
 struct DevBuf {
@@ -249,6 +251,9 @@ struct pgk_ctx {
   size_t hfw_xq_bytes = 0, hfw_cen_bytes = 0, hfw_mol_bytes = 0;
   double4 *d_hfw_v = nullptr;   // per slot: collision-part velocity (fused flux pass)
   size_t hfw_v_bytes = 0;
+  // volume mode's flux form: molecule and type per slot, the slots' sums
+  void *d_hfv_mt = nullptr, *d_hfv_acc = nullptr;
+  size_t hfv_mt_bytes = 0, hfv_acc_bytes = 0;
   int32_t *d_tl_start = nullptr, *d_tl_src = nullptr;
   uint32_t *d_tl_mask = nullptr;
   size_t tl_start_bytes = 0, tl_src_bytes = 0, tl_mask_bytes = 0;
@@ -431,6 +436,11 @@ static inline int pgk_grid_blocks(int64_t n, int bs) {
 // when the system has too few clusters to fill the device
 static inline bool pgk_pair_chunked(const pgk_ctx *c) {
   return (int64_t)c->ncl < c->pair_chunk_below;
+}
+
+static inline bool pgk_has_bonded(const pgk_ctx *c) {
+  return c->nbond_act > 0 || c->nangl_act > 0 || !c->tors_type.empty() || !c->rb_type.empty() ||
+         c->n14 > 0;
 }
 
 // waves of a pass over the current list in the form pgk_pair_chunked picks
