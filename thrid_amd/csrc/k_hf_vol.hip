@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void k_hf_pairs_vol(HfVolArgs p, HfDev h,
     int2 mj;
   };
   const int nent = e1 - e0;
-  bool any_inner = false;
+  bool any_inner = false, far = false;
   for (int cb = 0; cb < nent; cb += 64) {
     const int nin = min(64, nent - cb);
     const int c_hc = (lane < nin) ? p.cj[e0 + cb + lane] : 0;
@@ -278,12 +278,14 @@ __global__ __launch_bounds__(256) void k_hf_pairs_vol(HfVolArgs p, HfDev h,
 #pragma unroll
       for (int k = 0; k < 4; k++) so[k] = inner && same ? 0.0 : sj[k];
       const double t = hf_sum4x8(so, ii);
+      far = far || !(fabs(t) < 0x1p52);
       if (t != 0.0) vol_add(acc + (size_t)d.js * NW, ii >> 1, ii & 1, t);
       if (inner) {
         any_inner = true;
 #pragma unroll
         for (int k = 0; k < 4; k++) so[k] = same ? sj[k] : 0.0;
         const double u = hf_sum4x8(so, ii);
+        far = far || !(fabs(u) < 0x1p52);
         if (u != 0.0) vol_add(acc + (size_t)d.js * NW + NG, ii >> 1, ii & 1, u);
       }
     };
@@ -298,6 +300,10 @@ __global__ __launch_bounds__(256) void k_hf_pairs_vol(HfVolArgs p, HfDev h,
   }
   vol_add_i(acc + (size_t)islot * NW, si, lane >> 3);
   if (any_inner) vol_add_i(acc + (size_t)islot * NW + NG, sin, lane >> 3);
+  // a share that fixed point cannot hold (infinite, NaN): flagged for the
+  // regions' sums, which FP64 sums would carry it into
+  if (std::is_same<AH, unsigned long long>::value && __ballot(far) != 0 && lane == 0)
+    atomicOr(reinterpret_cast<unsigned long long *>(h.jpart) + 8 * (size_t)h.nreg, 1ull);
 }
 
 // one item's (slot's or atom's) contributions
@@ -463,6 +469,7 @@ __global__ __launch_bounds__(256) void k_hf_vol_final(HfBinArgs a, const double 
     if (src >= 0)
       for (int q = 0; q < G; q++) v += s[q][src];
     if (src >= 9) v += share_load(plane + ((size_t)r * 4 + (src - 9)) * 2);
+    if (src >= 9 && plane[8 * (size_t)a.nreg] != (AH)0) v = __builtin_nan("");
     if (k >= 9) v += acc_load(&jcol[3 * ((size_t)(k - 9) * a.nreg + r) + 2]);
     fin[k] = v * vol_inv;
   }
