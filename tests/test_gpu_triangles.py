@@ -1,6 +1,5 @@
-"""Triangle groups (rigid water) iterated on their separations: ordinary
-displacements, and ones large enough that the updates divide afresh in every
-sweep."""
+"""Triangle groups (rigid water): ordinary displacements, and ones comparable
+to a bond, whose sweeps start far from the constraints."""
 import numpy as np
 import pytest
 
@@ -11,8 +10,8 @@ import md_reference
 pytestmark = pytest.mark.gpu
 
 
-# 300 K: the quotient of an update changes by 0.1 % at most; 60000 K: by
-# more than the 5 % up to which its reciprocal is refined (checked below)
+# 300 K: a separation's projection on the old one changes by 0.1 % at most;
+# 60000 K: by a quarter (checked below)
 @pytest.mark.parametrize("temperature,far", [(300.0, False), (60000.0, True)])
 def test_triangle_sweeps_match_reference(oracle_mod, temperature, far):
     from thrid_amd.pgk import ForceContext

@@ -15,11 +15,8 @@
 // positions as rattle_c (rattle.F90:180-226), velocities as rattlep_v
 // (rattle_mtk.F90:455-490); divisions by quantities that stay constant
 // through the iteration are multiplications by reciprocals taken once.
-// Triangle groups run the same updates on their atoms' separations (a few
-// roundings from the reference's); other groups on the atoms themselves,
-// evaluated without contraction like the reference's build.
-#include <type_traits>
-
+// The sums are evaluated without contraction like the reference's build, but
+// for triangle groups' velocities and, in the FP64 form, positions.
 #include "pgk_device.h"
 
 
@@ -218,29 +215,29 @@ __device__ __forceinline__ bool rattle_one(const double3 &r, double rr2i, double
   return ok;
 }
 
-// 1/x from an estimate y of it (one Newton step: the relative error squares);
-// far is set where the estimate was too far off for that
-__device__ __forceinline__ double rcp_step(double x, double y, bool &far) {
-  const double e = __builtin_fma(-x, y, 1.0);
-  far = far || !(fabs(e) < 0.05);
-  return __builtin_fma(y, e, y);
+// num / x: the reciprocal's seed, one Newton step and one correction of the
+// quotient (relative error below 2^-52; x is no denormal here)
+__device__ __forceinline__ double quot(double num, double x) {
+  const double y0 = __builtin_amdgcn_rcp(x);
+  const double y = __builtin_fma(y0, __builtin_fma(-x, y0, 1.0), y0);
+  const double q = num * y;
+  return __builtin_fma(__builtin_fma(-x, q, num), y, q);
 }
 
 // a triangle group's position stage in registers: constraints (0,1), (0,2),
 // (1,2) in that order until an iteration moves nothing.
 // About 43 sweeps of three dependent updates: the chain of FP64 operations is
-// the time.  So the sweeps run on the two separations a = p0 - p1 and
-// b = p0 - p2 (p1 - p2 = b - a), whose change per update is one fused
-// multiply-add each, the multipliers of the old separations are summed, and
-// the three atoms move once at the end: the same updates and tests as
-// shake_one, about half the operations per
-// update.  The division by r . r_old keeps its reciprocal from sweep to sweep
-// and refines it by a Newton step, whose error is the square of the
-// quotient's change in one sweep; the last sweeps change it by less than the
-// tolerance, so their multipliers are exact to rounding.  A group whose
-// quotient jumps (a displacement comparable to a bond) divides in every
-// update instead.
-// First half step of 33,333 waters: 22.8 -> 17.4 us (1,693 waters: 20.0 -> 14.4).
+// the time.  FUSED, for FP64 forces, therefore contracts an update, divides in
+// six operations and leaves out the velocities, which follow once at the end
+// from the summed multipliers; a satisfied constraint divides zero by one (a
+// select of the quotient becomes a branch around the division, which then
+// waits for the test).  With FP32 forces the positions keep the reference's
+// roundings: a coordinate's last bit decides roundings of the FP32 spline
+// weights, and one of those changes the FFT's FP32 noise in every force, so a
+// trajectory would leave the unfused one's within steps.  (The shorter
+// division alone gains nothing there: 23.6 us against 23.0.)
+// First half step of 1,536 waters and 1,440 free atoms: 17.0 -> 13.4 us.
+template <bool FUSED>
 __device__ __forceinline__ bool shake_triangle(const ConsArgs &a, int c0, int i0, int i1, int i2,
                                                double3 &p0, double3 &p1, double3 &p2,
                                                double3 &v0, double3 &v1, double3 &v2,
@@ -250,79 +247,50 @@ __device__ __forceinline__ bool shake_triangle(const ConsArgs &a, int c0, int i0
   const double m0 = a.minv[i0], m1 = a.minv[i1], m2 = a.minv[i2];
   const double d01 = a.d2[c0], d02 = a.d2[c0 + 1], d12 = a.d2[c0 + 2];
   const double e01 = 1.0 / d01, e02 = 1.0 / d02, e12 = 1.0 / d12;
-  // multiplier = (r^2 - d^2) / (r . r_old) * h, h = 1 / (2 (1/mi + 1/mj))
-  const double m01 = m0 + m1, m02 = m0 + m2, m12 = m1 + m2;
-  const double h01 = 0.5 / m01, h02 = 0.5 / m02, h12 = 0.5 / m12;
-  double l01, l02, l12;
-  bool done;
-  auto sweeps = [&](auto divide) {
-    constexpr bool DIV = decltype(divide)::value;
-    double3 ra = sub(p0, p1), rb = sub(p0, p2);
-    double y01 = 1.0 / dot_f(ra, r01), y02 = 1.0 / dot_f(rb, r02),
-           y12 = 1.0 / dot_f(sub(rb, ra), r12);
-    bool far = false;
-    auto rcp = [&](double x, double &y) {
-      y = DIV ? 1.0 / x : rcp_step(x, y, far);
-      return y;
+  bool done = false;
+  if constexpr (FUSED) {
+    // multipliers of displacements (the reference's times dt)
+    double l01 = 0.0, l02 = 0.0, l12 = 0.0;
+    auto update = [&](double3 &pi, double3 &pj, const double3 &ro, double mi, double mj,
+                      double d2, double rd2, double &l) {
+      const double3 r = sub(pi, pj);
+      const double q = dot_f(r, r) - d2;
+      const bool ok = fabs(q) * rd2 < a.tol;
+      const double g = quot(ok ? 0.0 : 0.5 * q, ok ? 1.0 : dot_f(r, ro) * (mi + mj));
+      axpy(pi, -(mi * g), ro);
+      axpy(pj, mj * g, ro);
+      l += g;
+      return ok;
     };
-    l01 = l02 = l12 = 0.0;
-    done = false;
     for (int it = 0; it < a.maxit && !done; it++) {
-      {
-        const double q = dot_f(ra, ra) - d01;
-        const bool ok = fabs(q) * e01 < a.tol;
-        const double y = rcp(dot_f(ra, r01), y01);
-        const double g = ok ? 0.0 : (q * h01) * y;
-        axpy(ra, -(m01 * g), r01);
-        axpy(rb, -(m0 * g), r01);
-        l01 += g;
-        done = ok;
-      }
-      {
-        const double q = dot_f(rb, rb) - d02;
-        const bool ok = fabs(q) * e02 < a.tol;
-        const double y = rcp(dot_f(rb, r02), y02);
-        const double g = ok ? 0.0 : (q * h02) * y;
-        axpy(rb, -(m02 * g), r02);
-        axpy(ra, -(m0 * g), r02);
-        l02 += g;
-        done = ok && done;
-      }
-      {
-        const double3 rc = sub(rb, ra);
-        const double q = dot_f(rc, rc) - d12;
-        const bool ok = fabs(q) * e12 < a.tol;
-        const double y = rcp(dot_f(rc, r12), y12);
-        const double g = ok ? 0.0 : (q * h12) * y;
-        axpy(ra, m1 * g, r12);
-        axpy(rb, -(m2 * g), r12);
-        l12 += g;
-        done = ok && done;
-      }
+      done = update(p0, p1, r01, m0, m1, d01, e01, l01);
+      done = update(p0, p2, r02, m0, m2, d02, e02, l02) && done;
+      done = update(p1, p2, r12, m1, m2, d12, e12, l12) && done;
     }
-    return far;
-  };
-  if (sweeps(std::false_type{})) sweeps(std::true_type{});
-  // displacement of each atom, and the velocity it means over dt
-  const double idt = 1.0 / a.dt;
-  double3 s0 = make_double3(0.0, 0.0, 0.0), s1 = s0, s2 = s0;
-  axpy(s0, -(m0 * l01), r01);
-  axpy(s0, -(m0 * l02), r02);
-  axpy(s1, m1 * l01, r01);
-  axpy(s1, -(m1 * l12), r12);
-  axpy(s2, m2 * l02, r02);
-  axpy(s2, m2 * l12, r12);
-  axpy(p0, 1.0, s0);
-  axpy(p1, 1.0, s1);
-  axpy(p2, 1.0, s2);
-  axpy(v0, idt, s0);
-  axpy(v1, idt, s1);
-  axpy(v2, idt, s2);
+    const double idt = 1.0 / a.dt;
+    l01 *= idt;
+    l02 *= idt;
+    l12 *= idt;
+    axpy(v0, -(m0 * l01), r01);
+    axpy(v0, -(m0 * l02), r02);
+    axpy(v1, m1 * l01, r01);
+    axpy(v1, -(m1 * l12), r12);
+    axpy(v2, m2 * l02, r02);
+    axpy(v2, m2 * l12, r12);
+  } else {
+    for (int it = 0; it < a.maxit && !done; it++) {
+      done = shake_one(p0, p1, v0, v1, r01, m0, m1, d01, e01, a.tol, a.dt);
+      done = shake_one(p0, p2, v0, v2, r02, m0, m2, d02, e02, a.tol, a.dt) && done;
+      done = shake_one(p1, p2, v1, v2, r12, m1, m2, d12, e12, a.tol, a.dt) && done;
+    }
+  }
   return done;
 }
 
 // a triangle group's velocity stage in registers: the updates and tests of
-// rattle_one on the relative velocities v0 - v1 and v0 - v2, as above.
+// rattle_one on the relative velocities v0 - v1 and v0 - v2 (v1 - v2 is their
+// difference), whose change per update is one fused multiply-add each; the
+// multipliers are summed and the atoms take them once at the end.
 // Second half step of 33,333 waters: 15.3 -> 12.3 us (1,693 waters: 12.9 -> 10.3).
 __device__ __forceinline__ bool rattle_triangle(const ConsArgs &a, int c0, int i0, int i1,
                                                 int i2, const double3 &p0, const double3 &p1,
@@ -415,6 +383,7 @@ __device__ __forceinline__ void kick3(const double *force, const double *minv, i
 // When every group is a triangle: the first half step (kick, drift, position
 // constraints) in one pass, one thread per group, then one thread per atom
 // outside every group.  Same arithmetic as k_md_kick_drift + k_shake.
+template <bool FUSED>
 __global__ __launch_bounds__(64) void k_md_first_half(ConsArgs a, const double *__restrict__ force,
                                                       const int32_t *__restrict__ free_atoms,
                                                       int nfree) {
@@ -432,7 +401,7 @@ __global__ __launch_bounds__(64) void k_md_first_half(ConsArgs a, const double *
                 v1, o1, a.force_l, a.dt_l);
     kick_drift3(force, a.minv, i2, a.dt, kick_at(k, a.ltreg, a.vstrm, i2), p2,
                 v2, o2, a.force_l, a.dt_l);
-    const bool done = shake_triangle(a, c0, i0, i1, i2, p0, p1, p2, v0, v1, v2, o0, o1, o2);
+    const bool done = shake_triangle<FUSED>(a, c0, i0, i1, i2, p0, p1, p2, v0, v1, v2, o0, o1, o2);
     st3(a.pos, i0, p0);
     st3(a.pos, i1, p1);
     st3(a.pos, i2, p2);
@@ -479,6 +448,7 @@ __global__ __launch_bounds__(64) void k_md_second_half(ConsArgs a,
 }
 
 // positions (with the matching velocity correction), one group per thread
+template <bool FUSED>
 __global__ __launch_bounds__(64) void k_shake(ConsArgs a) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= a.ngroup) return;
@@ -489,7 +459,7 @@ __global__ __launch_bounds__(64) void k_shake(ConsArgs a) {
     double3 p0 = ld3(a.pos, i0), p1 = ld3(a.pos, i1), p2 = ld3(a.pos, i2);
     double3 v0 = ld3(a.vel, i0), v1 = ld3(a.vel, i1), v2 = ld3(a.vel, i2);
     const double3 o0 = ld3(a.pos_old, i0), o1 = ld3(a.pos_old, i1), o2 = ld3(a.pos_old, i2);
-    done = shake_triangle(a, c0, i0, i1, i2, p0, p1, p2, v0, v1, v2, o0, o1, o2);
+    done = shake_triangle<FUSED>(a, c0, i0, i1, i2, p0, p1, p2, v0, v1, v2, o0, o1, o2);
     st3(a.pos, i0, p0);
     st3(a.pos, i1, p1);
     st3(a.pos, i2, p2);
@@ -694,14 +664,15 @@ ConsArgs cons_args(pgk_ctx *c) {
 // over dt and the position constraints at dt
 int pgk_md_kick_drift(pgk_ctx *c, const double *f, double dt, const double *fl, double dtl) {
   const int n = c->natom;
+  const bool fused = c->precision == PGK_PREC_FP64;   // see shake_triangle
   ConsArgs a = cons_args(c);
   a.dt = dt;
   a.force_l = fl;
   a.dt_l = dtl;
   if (c->md_all_tri) {
     const int nt = c->md_ngroup + c->md_nfree;
-    k_md_first_half<<<pgk_grid_blocks(nt, 64), 64, 0, c->stream>>>(a, f, c->d_md_free,
-                                                                   c->md_nfree);
+    auto *k = fused ? k_md_first_half<true> : k_md_first_half<false>;
+    k<<<pgk_grid_blocks(nt, 64), 64, 0, c->stream>>>(a, f, c->d_md_free, c->md_nfree);
     HIP_CHECK(hipGetLastError());
     return pgk_md_strm_assign(c);   // at the new positions (moldyn_nhc.F90:1412)
   }
@@ -710,7 +681,8 @@ int pgk_md_kick_drift(pgk_ctx *c, const double *f, double dt, const double *fl, 
       a.vstrm);
   HIP_CHECK(hipGetLastError());
   if (c->md_ngroup > 0) {
-    k_shake<<<pgk_grid_blocks(c->md_ngroup, 64), 64, 0, c->stream>>>(a);
+    auto *k = fused ? k_shake<true> : k_shake<false>;
+    k<<<pgk_grid_blocks(c->md_ngroup, 64), 64, 0, c->stream>>>(a);
     HIP_CHECK(hipGetLastError());
   }
   return pgk_md_strm_assign(c);
