@@ -349,12 +349,26 @@ __device__ __forceinline__ void atom_frac_t(const double *pos, int i, const PmeG
   }
 }
 
+// The spreading bins: bin t holds the slots whose stencil starts in tile t at
+// items[start[t] .. start[t] + count[t]), up to start[t + 1]; slots that find
+// their bin full go to a list of their own (extra[0] counts them).  The starts
+// come from the counts at the last list build plus a margin (k_bin_start), so
+// between builds a call bins its slots in the preparation kernel itself, with
+// no scan and no second pass over the slots.  Those were two launches of 4-5
+// us in a chain that bounds small systems: 24,000 atoms in FP32 155 -> 146 us
+// per step, an 18,000-atom slab 169 -> 163, 5,079 atoms with heat flux 190 ->
+// 185.  An atom moves less than the list's margin between builds, under one
+// tile, so few slots overflow; each costs every tile one look.
+struct BinRef {
+  int32_t *count, *start, *items, *extra, *extra_items;
+};
+
 // Per-slot preparation ahead of the force kernels, in the list's spatial order
 // (order[k] = atom, or -1 for padding; identity without a list):
 //   - B-spline weights th[(d*P + q)*nitem + k] and the first stencil index
 //     base[k] = int(fr) - P + 1 per axis (get_bspline_coeffs and
 //     fill_charge_grid, fft_pme.F90:316-422), base.w = atom;
-//   - the slot's rank in its home tile bin: the block counts in LDS (open
+//   - the slot into its home tile bin: the block counts in LDS (open
 //     addressing on the tile id) and takes one global atomic per tile;
 //   - with PACK, the pair kernel's (x, y, z, q) and 0-based LJ type per slot.
 template <int PREC, int P, bool PACK>
@@ -365,8 +379,7 @@ __global__ __launch_bounds__(256) void k_prep(int nitem, const int32_t *__restri
                                               TileGeom tg,
                                               typename Prec<PREC>::real *__restrict__ th,
                                               int4 *__restrict__ base,
-                                              int32_t *__restrict__ count,
-                                              int32_t *__restrict__ rank,
+                                              BinRef bin,
                                               typename Prec<PREC>::real4 *__restrict__ xq,
                                               int32_t *__restrict__ ct) {
   using R = typename Prec<PREC>::real;
@@ -430,9 +443,35 @@ __global__ __launch_bounds__(256) void k_prep(int nitem, const int32_t *__restri
   }
   __syncthreads();
   for (int i = threadIdx.x; i < 512; i += blockDim.x)
-    if (s_key[i] >= 0) s_base[i] = atomicAdd(&count[s_key[i]], s_cnt[i]);
+    if (s_key[i] >= 0) s_base[i] = atomicAdd(&bin.count[s_key[i]], s_cnt[i]);
   __syncthreads();
-  if (k < nitem) rank[k] = (t >= 0) ? s_base[slot] + r : -1;
+  if (t >= 0) {
+    const int at = bin.start[t] + s_base[slot] + r;
+    if (at < bin.start[t + 1]) bin.items[at] = k;
+    else bin.extra_items[atomicAdd(bin.extra, 1)] = k;
+  }
+}
+
+// slots per bin at the current positions (the preparation kernel's binning),
+// for k_bin_start
+__global__ __launch_bounds__(256) void k_bin_count(int nitem, const int32_t *__restrict__ order,
+                                                   const double *__restrict__ pos, PmeGeom g,
+                                                   TileGeom tg, int32_t *__restrict__ count) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= nitem) return;
+  const int a = order ? order[k] : k;
+  if (a < 0) return;
+  int4 b;
+  int *bd = &b.x;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    double w = pos[3 * a + d] * g.recip[d];
+    w = w - floor(w);
+    double fr = (double)g.K[d] * w;
+    if (!(fr >= 0.0 && fr < (double)g.K[d])) fr = (fr >= (double)g.K[d]) ? (double)g.K[d] - 1.0 : 0.0;
+    bd[d] = (int)fr - g.order + 1;
+  }
+  atomicAdd(&count[tile_home(b, g, tg)], 1);
 }
 
 // Forces from the potential grid (grad_sum, fft_pme.F90:515-590): four
@@ -446,9 +485,13 @@ __global__ __launch_bounds__(256) void k_gather_t(int nitem, const int32_t *__re
                                                   const double *__restrict__ q, PmeGeom g,
                                                   const void *gridv,
                                                   typename Prec<PREC>::acc *fat,
-                                                  typename Prec<PREC>::acc *fat_c) {
+                                                  typename Prec<PREC>::acc *fat_c, BinRef bin,
+                                                  int ntile) {
   using R = typename Prec<PREC>::real;
   const int t = xcd_block() * blockDim.x + threadIdx.x;
+  // the spreading is done: the bins start empty at the next call
+  for (int z = t; z < ntile; z += gridDim.x * blockDim.x) bin.count[z] = 0;
+  if (t == 0) bin.extra[0] = 0;
   const int k = t >> 2, sub = t & 3;
   // whole groups of four lanes leave together, so the shuffles below see
   // their partners
@@ -559,15 +602,17 @@ __global__ __launch_bounds__(256) void k_phi_atoms(int n, const double *__restri
 // One workgroup per tile accumulates the points it owns in LDS (int64 fixed
 // point in the mixed form: order-independent) and writes each grid point
 // once, in the compute type.  No device atomics, no clearing pass.
-// exclusive scan of count[0..n) into start[0..n] (start[n] = total), one
-// block: each thread sums a contiguous chunk, the block scans the chunk sums
-__global__ __launch_bounds__(1024) void k_scan_start(int n, const int32_t *__restrict__ count,
-                                                     int32_t *__restrict__ start) {
+// starts of the bins: each has room for half as many slots again as it holds
+// now, and 16 more (one block: each thread sums a contiguous chunk, the block
+// scans the chunk sums); the counts are left at zero for the next preparation
+__device__ __host__ __forceinline__ int bin_room(int n) { return n + n / 2 + 16; }
+__global__ __launch_bounds__(1024) void k_bin_start(int n, int32_t *__restrict__ count,
+                                                    int32_t *__restrict__ start) {
   __shared__ int s[1024];
   const int per = (n + 1023) / 1024;
   const int lo = min((int)threadIdx.x * per, n), hi = min(lo + per, n);
   int sum = 0;
-  for (int i = lo; i < hi; i++) sum += count[i];
+  for (int i = lo; i < hi; i++) sum += bin_room(count[i]);
   s[threadIdx.x] = sum;
   __syncthreads();
   for (int off = 1; off < 1024; off <<= 1) {
@@ -579,25 +624,10 @@ __global__ __launch_bounds__(1024) void k_scan_start(int n, const int32_t *__res
   int run = s[threadIdx.x] - sum;
   for (int i = lo; i < hi; i++) {
     start[i] = run;
-    run += count[i];
+    run += bin_room(count[i]);
+    count[i] = 0;
   }
   if (threadIdx.x == 1023) start[n] = s[1023];
-}
-
-// items of every bin in rank order; the counts (already scanned) are left
-// zeroed for the next call's k_prep
-__global__ __launch_bounds__(256) void k_tile_fill(int nitem, const int4 *__restrict__ base,
-                                                   PmeGeom g, TileGeom tg,
-                                                   int32_t *__restrict__ count,
-                                                   const int32_t *__restrict__ start,
-                                                   const int32_t *__restrict__ rank,
-                                                   int32_t *__restrict__ items) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int z = k; z < tg.ntile; z += gridDim.x * blockDim.x) count[z] = 0;
-  if (k >= nitem) return;
-  const int r = rank[k];
-  if (r < 0) return;
-  items[start[tile_home(base[k], g, tg)] + r] = k;
 }
 
 template <int PREC> struct SpreadAcc { using type = typename Prec<PREC>::real; };
@@ -629,8 +659,7 @@ __device__ __forceinline__ unsigned stencil_bits(int b, int o, int T, int K) {
 template <int PREC, int P>
 __global__ __launch_bounds__(64) void k_spread_tile(int nitem, const double *__restrict__ q,
                                                     PmeGeom g, TileGeom tg,
-                                                    const int32_t *__restrict__ start,
-                                                    const int32_t *__restrict__ items,
+                                                    BinRef bn,
                                                     const typename Prec<PREC>::real *__restrict__ th,
                                                     const int4 *__restrict__ base,
                                                     typename Prec<PREC>::real *__restrict__ grid) {
@@ -658,9 +687,11 @@ __global__ __launch_bounds__(64) void k_spread_tile(int nitem, const double *__r
     const int sy = (ty - dy + tg.nt[1]) % tg.nt[1];
     const int sz = (tz - dz + tg.nt[2]) % tg.nt[2];
     const int bin = (sz * tg.nt[1] + sy) * tg.nt[0] + sx;
-    s_lo[u] = start[bin];
-    s_n[u + 1] = start[bin + 1] - start[bin];
+    const int b0 = bn.start[bin];
+    s_lo[u] = b0;
+    s_n[u + 1] = min(bn.count[bin], bn.start[bin + 1] - b0);
   }
+  const int nextra = bn.extra[0];   // slots whose bin was full: seen by every tile
   if (lane == 0) s_nv = 0;
   __syncthreads();
   if (lane == 0) {
@@ -668,13 +699,17 @@ __global__ __launch_bounds__(64) void k_spread_tile(int nitem, const double *__r
     for (int u = 0; u < nsrc; u++) s_n[u + 1] += s_n[u];
   }
   __syncthreads();
-  const int total = s_n[nsrc];
+  const int nbin = s_n[nsrc], total = nbin + nextra;
+  auto visit = [&](int v) {   // the slot of visit v
+    if (v >= nbin) return bn.extra_items[v - nbin];
+    int u = 0;
+    while (u + 1 < nsrc && v >= s_n[u + 1]) u++;
+    return bn.items[s_lo[u] + (v - s_n[u])];
+  };
   // keep the visits whose stencil meets the tile (the kept order does not
   // matter: the additions below commute exactly in the mixed form)
   for (int v = lane; v < total; v += 64) {
-    int u = 0;
-    while (u + 1 < nsrc && v >= s_n[u + 1]) u++;
-    const int k = items[s_lo[u] + (v - s_n[u])];
+    const int k = visit(v);
     const int4 b = base[k];
     if (stencil_bits<P>(b.x, ox, T0, g.K[0]) && stencil_bits<P>(b.y, oy, T1, g.K[1]) &&
         stencil_bits<P>(b.z, oz, T2, g.K[2])) {
@@ -693,10 +728,7 @@ __global__ __launch_bounds__(64) void k_spread_tile(int nitem, const double *__r
     if (w < nv) {
       k = s_vis[w];
     } else {
-      const int v = w - nv;
-      int u = 0;
-      while (u + 1 < nsrc && v >= s_n[u + 1]) u++;
-      k = items[s_lo[u] + (v - s_n[u])];
+      k = visit(w - nv);
       bool listed = false;
       for (int x = 0; x < nv && !listed; x++) listed = s_vis[x] == k;
       if (listed) continue;
@@ -1585,7 +1617,7 @@ struct PmeLayout {
   const int32_t *order;
   void *th;
   int4 *base;
-  int32_t *count, *start, *rank, *items;
+  BinRef bin;
 };
 
 static int pme_layout(pgk_ctx *c, size_t rsize, PmeLayout *L) {
@@ -1628,8 +1660,10 @@ static int pme_layout(pgk_ctx *c, size_t rsize, PmeLayout *L) {
   L->th = c->d_theta;
   L->base = reinterpret_cast<int4 *>(reinterpret_cast<char *>(c->d_theta) +
                                      nitem * 3 * c->order * rsize);
-  // bins: count[ntile] | start[ntile + 1] | rank[nitem] | items[nitem]
-  size_t tneed = sizeof(int32_t) * (2 * (size_t)tg.ntile + 1 + 2 * nitem);
+  // bins: count[ntile] | extra count | start[ntile + 1] | extra items[nitem] |
+  // items (the bins' room)
+  const size_t room = nitem + nitem / 2 + 16 * (size_t)tg.ntile;
+  const size_t tneed = sizeof(int32_t) * (2 * (size_t)tg.ntile + 2 + nitem + room);
   if (tneed > c->tile_bytes || c->tile_ntile != tg.ntile) {
     if (c->d_tile) (void)hipFree(c->d_tile);
     c->d_tile = nullptr;
@@ -1637,13 +1671,15 @@ static int pme_layout(pgk_ctx *c, size_t rsize, PmeLayout *L) {
     HIP_CHECK(hipMalloc(&c->d_tile, tneed));
     c->tile_bytes = tneed;
     c->tile_ntile = tg.ntile;
-    // counts start at zero; afterwards k_tile_fill leaves them zeroed
-    HIP_CHECK(hipMemsetAsync(c->d_tile, 0, sizeof(int32_t) * tg.ntile, c->stream));
+    c->tile_serial = -1;
+    // counts start at zero; afterwards k_gather_t leaves them zeroed
+    HIP_CHECK(hipMemsetAsync(c->d_tile, 0, sizeof(int32_t) * (tg.ntile + 1), c->stream));
   }
-  L->count = reinterpret_cast<int32_t *>(c->d_tile);
-  L->start = L->count + tg.ntile;
-  L->rank = L->start + tg.ntile + 1;
-  L->items = L->rank + nitem;
+  L->bin.count = reinterpret_cast<int32_t *>(c->d_tile);
+  L->bin.extra = L->bin.count + tg.ntile;
+  L->bin.start = L->bin.extra + 1;
+  L->bin.extra_items = L->bin.start + tg.ntile + 1;
+  L->bin.items = L->bin.extra_items + nitem;
   return PGK_OK;
 }
 
@@ -1655,12 +1691,23 @@ int launch_prep(pgk_ctx *c) {
   int rc = pme_layout(c, sizeof(R), &L);
   if (rc) return rc;
   const int gb = pgk_grid_blocks(L.nitem, 256);
+  // the bins' starts follow the list: a rebuild changes the slots and comes
+  // where the atoms have moved; without a list (charges alone) nothing bounds
+  // the motion between calls and each call takes new ones
+  if (!L.order || c->tile_serial != c->list_serial || c->tile_nitem != L.nitem) {
+    k_bin_count<<<gb, 256, 0, c->stream>>>(L.nitem, L.order, c->d_pos, L.g, L.tg, L.bin.count);
+    HIP_CHECK(hipGetLastError());
+    k_bin_start<<<1, 1024, 0, c->stream>>>(L.tg.ntile, L.bin.count, L.bin.start);
+    HIP_CHECK(hipGetLastError());
+    c->tile_serial = L.order ? c->list_serial : -1;
+    c->tile_nitem = L.nitem;
+  }
   R *th = reinterpret_cast<R *>(L.th);
   R4 *xq = reinterpret_cast<R4 *>(c->d_xq);
 #define PGK_PREP(P)                                                                          \
   k_prep<PREC, P, PACK><<<gb, 256, 0, c->stream>>>(L.nitem, L.order, c->d_pos, c->d_q,      \
-                                                   c->d_type, L.g, L.tg, th, L.base, L.count, \
-                                                   L.rank, xq, c->d_ct)
+                                                   c->d_type, L.g, L.tg, th, L.base, L.bin,  \
+                                                   xq, c->d_ct)
   switch (c->order) {
     case 3: PGK_PREP(3); break;
     case 4: PGK_PREP(4); break;
@@ -1694,15 +1741,11 @@ int launch_pme(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
   int4 *base = L.base;
   pgk_prof_begin(c, PGK_PROF_SPREAD);
   {
-    k_scan_start<<<1, 1024, 0, st>>>(tg.ntile, L.count, L.start);
-    k_tile_fill<<<pgk_grid_blocks(std::max(nitem, tg.ntile), 256), 256, 0, st>>>(
-        nitem, base, g, tg, L.count, L.start, L.rank, L.items);
     const size_t lds = (size_t)tg.T[0] * tg.T[1] * tg.T[2] * sizeof(typename SpreadAcc<PREC>::type);
     R *gr = reinterpret_cast<R *>(c->d_grid);
-    const int32_t *start = L.start, *items = L.items;
 #define PGK_SPREAD(P)                                                                         \
-  k_spread_tile<PREC, P><<<xcd_grid(tg.ntile), 64, lds, st>>>(nitem, c->d_q, g, tg, start,    \
-                                                                items, th, base, gr)
+  k_spread_tile<PREC, P><<<xcd_grid(tg.ntile), 64, lds, st>>>(nitem, c->d_q, g, tg, L.bin, th, \
+                                                                base, gr)
     switch (c->order) {
       case 3: PGK_SPREAD(3); break;
       case 4: PGK_SPREAD(4); break;
@@ -1826,7 +1869,7 @@ int launch_pme(pgk_ctx *c, bool split, bool ene, int *off, int *nrec) {
     const int gbx = xcd_grid(gb);
 #define PGK_GATHER(SP, P)                                                                 \
   k_gather_t<PREC, SP, P><<<gbx, 256, 0, st>>>(nitem, ord, c->d_pos, c->d_q, g, c->d_pgrid, \
-                                              fat, fatc)
+                                              fat, fatc, L.bin, tg.ntile)
     const int32_t *ord = L.order;
     if (split) {
       switch (c->order) {

@@ -302,7 +302,7 @@ int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom
       HIP_CHECK(hipMemsetAsync(c->d_fcl_c, 0, nsc * 3 * ab, st));
     }
     if (c->d_tile && c->tile_ntile > 0)   // spreading bin counts
-      HIP_CHECK(hipMemsetAsync(c->d_tile, 0, sizeof(int32_t) * c->tile_ntile, st));
+      HIP_CHECK(hipMemsetAsync(c->d_tile, 0, sizeof(int32_t) * (c->tile_ntile + 1), st));
   }
   c->acc_dirty = true;
   const bool do_ewk = (m->ewk == mts_flag);

@@ -226,9 +226,10 @@ struct pgk_ctx {
   void *d_cgrid = nullptr;         // complex half grid ((n1/2+1)*n2*n3)
   void *d_theta = nullptr;         // B-spline weights + base indices per atom
   size_t theta_bytes = 0;
-  void *d_tile = nullptr;          // spreading bins: counts, starts, ranks, items, scan space
+  void *d_tile = nullptr;          // spreading bins: counts, starts, items
   size_t tile_bytes = 0;
-  int tile_ntile = 0;
+  int tile_ntile = 0, tile_nitem = 0;
+  int64_t tile_serial = -1;        // the list build the bins' starts are of
   double *d_tw = nullptr;          // twiddles: 3 dims, each n complex (FP64)
   float *d_twf = nullptr;
   int tw_off[3] = {0, 0, 0};
