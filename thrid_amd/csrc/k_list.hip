@@ -13,6 +13,9 @@
 // 2 cj + h and a 32-bit mask whose bit (ii + 8 jq) records the reference's
 // decision for the pair (i-slot ii, j-slot 4 h + jq).  The pair kernel
 // evaluates exactly the masked pairs, two entries per wavefront pass.
+#include <algorithm>
+#include <cstdint>
+
 #include <hipcub/hipcub.hpp>
 
 #include "pgk_internal.h"
@@ -77,61 +80,110 @@ __global__ void k_sort_bins(int nbin, const int32_t *__restrict__ bin_start,
   }
 }
 
-__global__ void k_col_counts(int ncolumn, int nzb, const int32_t *__restrict__ bin_start,
-                             int32_t *__restrict__ col_ncl) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncolumn) return;
-  int cnt = bin_start[(c + 1) * nzb] - bin_start[c * nzb];
-  col_ncl[c] = (cnt + PGK_CL - 1) / PGK_CL;
-}
-
-// one block per column
-__global__ void k_fill_clusters(int nzb, const int32_t *__restrict__ bin_start,
-                                const int32_t *__restrict__ sorted,
-                                const int32_t *__restrict__ col_ncl,
-                                const int32_t *__restrict__ col_clstart,
-                                int32_t *__restrict__ cl_atom,
-                                int32_t *__restrict__ cl_col,
-                                int32_t *__restrict__ slot_of) {
-  int c = blockIdx.x;
-  int s0 = bin_start[c * nzb];
-  int cnt = bin_start[(c + 1) * nzb] - s0;
-  int nslot = col_ncl[c] * PGK_CL;
-  int base = col_clstart[c] * PGK_CL;
-  for (int k = threadIdx.x; k < nslot; k += blockDim.x) {
-    int a = (k < cnt) ? sorted[s0 + k] : -1;
-    cl_atom[base + k] = a;
-    if (a >= 0) slot_of[a] = base + k;
-    if ((k & (PGK_CL - 1)) == 0) cl_col[col_clstart[c] + k / PGK_CL] = c;
-  }
-}
-
-// bounding boxes of the clusters (wrapped frame) and the slots' FP64
-// positions with the atom index in .w (-1 for padding), for the pair search
-__global__ void k_bbox(const int32_t *__restrict__ ncl, const double *__restrict__ pos,
-                       const int32_t *__restrict__ cl_atom, GridGeom g,
-                       float *__restrict__ bbox, double4 *__restrict__ posc) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= *ncl) return;
-  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  for (int k = 0; k < PGK_CL; k++) {
-    int a = cl_atom[c * PGK_CL + k];
-    posc[c * PGK_CL + k] = (a >= 0) ? make_double4(pos[3 * a], pos[3 * a + 1], pos[3 * a + 2],
-                                                   (double)a)
-                                    : make_double4(0.0, 0.0, 0.0, -1.0);
-    if (a < 0) continue;
-    for (int d = 0; d < 3; d++) {
-      double w = wrap_coord(pos[3 * a + d], g.L[d]);
-      lo[d] = fmin(lo[d], w);
-      hi[d] = fmax(hi[d], w);
+// exclusive scan of value(0 .. n) with store(k, before k) and the total, one
+// block of 1024: tiles of 4 elements a thread, the running sum carried along
+template <class V, class S>
+__device__ __forceinline__ uint64_t block_scan(int n, V value, S store) {
+  __shared__ uint64_t s_sum[16];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  uint64_t carry = 0;
+  for (int k0 = 0; k0 < n; k0 += 4096) {
+    const int k = k0 + 4 * t;
+    uint64_t v[4], own = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      v[q] = (k + q < n) ? value(k + q) : 0;
+      own += v[q];
+    }
+    uint64_t incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint64_t up = __shfl_up(incl, o);
+      if (lane >= o) incl += up;
+    }
+    __syncthreads();   // the last tile's sums are read
+    if (lane == 63) s_sum[wave] = incl;
+    __syncthreads();
+    uint64_t run = carry + incl - own;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+      const uint64_t sw = s_sum[w];
+      if (w < wave) run += sw;
+      carry += sw;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (k + q < n) store(k + q, run);
+      run += v[q];
     }
   }
-  for (int d = 0; d < 3; d++) {
-    bbox[c * 8 + d] = (float)lo[d] - 1e-3f;
-    bbox[c * 8 + 4 + d] = (float)hi[d] + 1e-3f;
+  return carry;
+}
+
+// clusters of every column and their first cluster, one block; clears the
+// search's overflow flags
+__global__ __launch_bounds__(1024) void k_col_scan(int ncolumn, int nzb,
+                                                   const int32_t *__restrict__ bin_start,
+                                                   int32_t *__restrict__ col_ncl,
+                                                   int32_t *__restrict__ col_clstart,
+                                                   int32_t *__restrict__ overflow) {
+  const uint64_t tot = block_scan(
+      ncolumn,
+      [&](int c) {
+        const int cnt = bin_start[(c + 1) * nzb] - bin_start[c * nzb];
+        const int ncl = (cnt + PGK_CL - 1) / PGK_CL;
+        col_ncl[c] = ncl;
+        return (uint64_t)ncl;
+      },
+      [&](int c, uint64_t at) { col_clstart[c] = (int32_t)at; });
+  if (threadIdx.x == 0) {
+    col_clstart[ncolumn] = (int32_t)tot;
+    *overflow = 0;
   }
-  bbox[c * 8 + 3] = 0.f;
-  bbox[c * 8 + 7] = 0.f;
+}
+
+// one block per column: the clusters' slots, the slots' FP64 positions with
+// the atom index in .w (-1 for padding) and the clusters' bounding boxes
+// (wrapped frame) for the pair search.  Eight lanes share a cluster.
+__global__ __launch_bounds__(64) void k_fill_clusters(
+    GridGeom g, const int32_t *__restrict__ bin_start, const int32_t *__restrict__ sorted,
+    const int32_t *__restrict__ col_ncl, const int32_t *__restrict__ col_clstart,
+    const double *__restrict__ pos, int32_t *__restrict__ cl_atom, int32_t *__restrict__ cl_col,
+    int32_t *__restrict__ slot_of, float *__restrict__ bbox, double4 *__restrict__ posc) {
+  const int c = blockIdx.x;
+  const int s0 = bin_start[c * g.nzb];
+  const int cnt = bin_start[(c + 1) * g.nzb] - s0;
+  const int nslot = col_ncl[c] * PGK_CL;
+  const int base = col_clstart[c] * PGK_CL;
+  for (int k = threadIdx.x; k < nslot; k += 64) {   // whole clusters: no lane leaves its eight
+    const int a = (k < cnt) ? sorted[s0 + k] : -1;
+    double p[3] = {0.0, 0.0, 0.0};
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    cl_atom[base + k] = a;
+    if (a >= 0) {
+      slot_of[a] = base + k;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        p[d] = pos[3 * a + d];
+        lo[d] = hi[d] = wrap_coord(p[d], g.L[d]);
+      }
+    }
+    posc[base + k] = make_double4(p[0], p[1], p[2], (double)a);
+#pragma unroll
+    for (int o = 1; o < PGK_CL; o <<= 1)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        lo[d] = fmin(lo[d], __shfl_xor(lo[d], o));
+        hi[d] = fmax(hi[d], __shfl_xor(hi[d], o));
+      }
+    if ((k & (PGK_CL - 1)) == 0) {
+      const int cl = base / PGK_CL + k / PGK_CL;
+      cl_col[cl] = c;
+      float4 *b = reinterpret_cast<float4 *>(bbox + (size_t)cl * 8);
+      b[0] = make_float4((float)lo[0] - 1e-3f, (float)lo[1] - 1e-3f, (float)lo[2] - 1e-3f, 0.f);
+      b[1] = make_float4((float)hi[0] + 1e-3f, (float)hi[1] + 1e-3f, (float)hi[2] + 1e-3f, 0.f);
+    }
+  }
 }
 
 // minimal periodic gap between intervals [a0,a1] and [b0,b1] in a box of length L
@@ -149,12 +201,18 @@ __device__ __forceinline__ float pgap(float a0, float a1, float b0, float b1, fl
 // packed positions: the minimum-image r^2 does not depend on which atom comes
 // first (IEEE subtraction and round() are odd functions), so the slot order
 // can be used
+// WIDE: the box is wider than twice the cutoff, and a tie of round() (|r| half
+// a box length either way) is no pair, so the one-instruction rint() will do.
+template <bool WIDE>
 __device__ __forceinline__ bool ref_pair_in4(const double4 &p, const double4 &q, const double *L,
                                              const double *Linv, double sqcut) {
 #pragma clang fp contract(off)
   double r[3] = {p.x - q.x, p.y - q.y, p.z - q.z};
 #pragma unroll
-  for (int d = 0; d < 3; d++) r[d] = r[d] - L[d] * round(r[d] * Linv[d]);
+  for (int d = 0; d < 3; d++) {
+    const double n = r[d] * Linv[d];
+    r[d] = r[d] - L[d] * (WIDE ? rint(n) : round(n));
+  }
   double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
   return r2 < sqcut;
 }
@@ -181,7 +239,7 @@ struct ListArgs {
   uint32_t *tmp_mask;
   int32_t *ci_count;
   int32_t *overflow;
-  int ncolumn, ncl_max;
+  int ncolumn;
   int ncol[2], rng[2];
   double L[3], Linv[3];
   float Lf[3], colwf[2];
@@ -204,30 +262,39 @@ __device__ __forceinline__ int zsearch(const float *__restrict__ bbox, int c0, i
   return lo;
 }
 
-// One wavefront per i-cluster.
+// One block of PGK_FW waves per i-cluster.
 // Phase A walks the x-y columns within reach, at or after the i-cluster's own
 // column (cluster indices are column-major, and only cj >= ci is kept).  For
 // each column one lane finds by binary search the clusters whose z range can
 // come within rcut_book of the i-cluster's box (a circular window when the
 // reach crosses the periodic z boundary); the windows of up to 64 columns are
-// then tested 64 clusters at a time with the bounding-box gap, and survivors
-// are compacted into LDS.
+// then tested with the bounding-box gap, 64 clusters a wave, and survivors are
+// compacted into LDS in the windows' order.
 // Phase B decides every atom pair of every surviving cluster pair with the
 // reference's exact FP64 test, lane = ii + 8*jj, PGK_UNROLL candidates per
-// iteration, and writes (cj, 64-bit mask) for nonzero masks.
-// NW waves per block: 4, or 1 for small systems, whose few clusters then
-// spread over all CUs instead of a quarter as many blocks
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_find_pairs(ListArgs a) {
-  __shared__ int32_t s_cand[NW][PGK_MAXJ];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int ci = blockIdx.x * NW + wave;
-  const int ncl = a.col_clstart[a.ncolumn];
-  const bool active = ci < ncl;
-  int32_t *cand = s_cand[wave];
+// iteration and wave, into 64-bit masks in LDS.
+// Phase C compacts the nonzero half masks, a share of the candidates per wave,
+// in the candidates' order.
+// A cluster's search is a chain of dependent loads and shuffles, and a system
+// of a few thousand clusters has fewer than the device holds waves: with one
+// wave per cluster and no list of masks 1,693 waters took 106 us, an
+// 18,000-atom slab 212 and 33,333 waters 262; now 21, 70 and 161 (8, 10 and 10
+// of them by rint, see ref_pair_in4, and the exclusions' range).
+#define PGK_FW 4
+// WIDE: every box length beyond twice the cutoff (see ref_pair_in4; a build
+// with the cutoff above half the box is refused, so only equality is not)
+template <bool WIDE>
+__global__ __launch_bounds__(64 * PGK_FW) void k_find_pairs(ListArgs a) {
+  __shared__ int32_t cand[PGK_MAXJ];
+  __shared__ uint64_t s_mask[PGK_MAXJ];
+  __shared__ int s_cnt[2][PGK_FW];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ci = blockIdx.x;
+  if (ci >= a.col_clstart[a.ncolumn]) return;
+  const uint64_t below = (1ull << lane) - 1ull;
   bool ovf = false;
   int ncand = 0;
-  if (active) {
+  {
     const float4 blo = *reinterpret_cast<const float4 *>(a.bbox + ci * 8);
     const float4 bhi = *reinterpret_cast<const float4 *>(a.bbox + ci * 8 + 4);
     const float ilo[3] = {blo.x, blo.y, blo.z}, ihi[3] = {bhi.x, bhi.y, bhi.z};
@@ -251,6 +318,7 @@ __global__ __launch_bounds__(64 * NW) void k_find_pairs(ListArgs a) {
       ze -= a.Lf[2];
     }
     const int nwin = nx * ny;
+    int turn = 0;
     for (int w0 = 0; w0 < nwin; w0 += 64) {
       const int w = w0 + lane;
       int c0 = 0, cn = 0, start = 0, len = 0;
@@ -289,10 +357,10 @@ __global__ __launch_bounds__(64 * NW) void k_find_pairs(ListArgs a) {
       }
       const int off = incl - len;
       const int total = __shfl(incl, 63);
-      for (int t0 = 0; t0 < total; t0 += 64) {
+      for (int t0 = 0; t0 < total; t0 += 64 * PGK_FW, turn ^= 1) {
         // every lane runs the shuffles (a shuffle from an inactive lane reads
         // nothing useful); lanes past the end repeat the last element
-        const int t = t0 + lane;
+        const int t = t0 + 64 * wave + lane;
         const int tt = min(t, total - 1);
         int lo = 0;   // the window holding tt: the last lane whose offset is <= tt
 #pragma unroll
@@ -306,29 +374,39 @@ __global__ __launch_bounds__(64 * NW) void k_find_pairs(ListArgs a) {
         const int cj = wc0 + k;
         bool pass = false;
         if (t < total && cj >= ci) {
-          const float4 jlo = *reinterpret_cast<const float4 *>(a.bbox + cj * 8);
-          const float4 jhi = *reinterpret_cast<const float4 *>(a.bbox + cj * 8 + 4);
+          const float4 jlo = *reinterpret_cast<const float4 *>(a.bbox + (size_t)cj * 8);
+          const float4 jhi = *reinterpret_cast<const float4 *>(a.bbox + (size_t)cj * 8 + 4);
           const float g0 = pgap(ilo[0], ihi[0], jlo.x, jhi.x, a.Lf[0]);
           const float g1 = pgap(ilo[1], ihi[1], jlo.y, jhi.y, a.Lf[1]);
           const float g2 = pgap(ilo[2], ihi[2], jlo.z, jhi.z, a.Lf[2]);
           pass = g0 * g0 + g1 * g1 + g2 * g2 < a.rcbf2;
         }
         const uint64_t bal = __ballot(pass);
-        const int pos = __popcll(bal & ((1ull << lane) - 1ull));
+        // the two sets of counts take turns, so one barrier a turn will do
+        if (lane == 0) s_cnt[turn][wave] = (int)__popcll(bal);
+        __syncthreads();
+        int at = ncand + (int)__popcll(bal & below), sum = 0;
+#pragma unroll
+        for (int w2 = 0; w2 < PGK_FW; w2++) {
+          const int n2 = s_cnt[turn][w2];
+          if (w2 < wave) at += n2;
+          sum += n2;
+        }
         if (pass) {
-          if (ncand + pos < PGK_MAXJ) cand[ncand + pos] = cj;
+          if (at < PGK_MAXJ) cand[at] = cj;
           else ovf = true;
         }
-        ncand = min(ncand + (int)__popcll(bal), PGK_MAXJ);
+        ncand = min(ncand + sum, PGK_MAXJ);
       }
     }
   }
   __syncthreads();
-  if (active) {
+  {
     const int ii = lane & 7, jj = lane >> 3;
-    const double4 pi4 = a.posc[ci * PGK_CL + ii];
+    const double4 pi4 = a.posc[(size_t)ci * PGK_CL + ii];
     const int ai = (int)pi4.w;
-    int xp[PGK_XREG];
+    // exclusion partners, and their range: few candidates fall into it
+    int xp[PGK_XREG], xlo = INT32_MAX, xhi = -1;
     bool xmem = false;
     {
       int s0 = 0, nxp = 0;
@@ -338,109 +416,136 @@ __global__ __launch_bounds__(64 * NW) void k_find_pairs(ListArgs a) {
       }
       xmem = nxp > PGK_XREG;
 #pragma unroll
-      for (int q = 0; q < PGK_XREG; q++) xp[q] = (q < nxp) ? a.xs_j[s0 + q] : -1;
+      for (int q = 0; q < PGK_XREG; q++) {
+        xp[q] = (q < nxp) ? a.xs_j[s0 + q] : -1;
+        if (q < nxp) {
+          xlo = min(xlo, xp[q]);
+          xhi = max(xhi, xp[q]);
+        }
+      }
+      if (xmem) {
+        xlo = 0;
+        xhi = INT32_MAX;
+      }
     }
-    int count = 0;
-    for (int k0 = 0; k0 < ncand; k0 += PGK_UNROLL) {
+    for (int k0 = wave * PGK_UNROLL; k0 < ncand; k0 += PGK_FW * PGK_UNROLL) {
       int cjv[PGK_UNROLL];
       double4 pj[PGK_UNROLL];
 #pragma unroll
       for (int u = 0; u < PGK_UNROLL; u++) {
         cjv[u] = cand[min(k0 + u, ncand - 1)];
-        pj[u] = a.posc[cjv[u] * PGK_CL + jj];
+        pj[u] = a.posc[(size_t)cjv[u] * PGK_CL + jj];
       }
 #pragma unroll
       for (int u = 0; u < PGK_UNROLL; u++) {
         if (k0 + u >= ncand) break;
-        const int cj = cjv[u];
         const int aj = (int)pj[u].w;
-        bool in = false;
-        if (ai >= 0 && aj >= 0 && (cj != ci || ii < jj)) {
-          in = ref_pair_in4(pi4, pj[u], a.L, a.Linv, a.sqcut);
-          if (in) {
-            bool ex = false;
+        bool in = ref_pair_in4<WIDE>(pi4, pj[u], a.L, a.Linv, a.sqcut) && ai >= 0 && aj >= 0 &&
+                  (cjv[u] != ci || ii < jj);
+        if (in && aj >= xlo && aj <= xhi) {
+          bool ex = false;
 #pragma unroll
-            for (int q = 0; q < PGK_XREG; q++) ex = ex || (xp[q] == aj);
-            if (xmem) ex = excluded(a.xidx, a.xlst, ai, aj);
-            in = !ex;
-          }
+          for (int q = 0; q < PGK_XREG; q++) ex = ex || (xp[q] == aj);
+          if (xmem) ex = excluded(a.xidx, a.xlst, ai, aj);
+          in = !ex;
         }
         const uint64_t m = __ballot(in);
-        // one entry per half j-cluster with a listed pair: slots jj = 0..3
-        // (mask bits 0..31) and jj = 4..7 (bits 32..63)
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-          const uint32_t mh = (uint32_t)(m >> (32 * hh));
-          if (mh) {
-            if (lane == 0) {
-              if (count < PGK_MAXJ) {
-                a.tmp_cj[(size_t)ci * PGK_MAXJ + count] = 2 * cj + hh;
-                a.tmp_mask[(size_t)ci * PGK_MAXJ + count] = mh;
-              } else {
-                ovf = true;
-              }
-            }
-            count++;
-          }
-        }
+        if (lane == 0) s_mask[k0 + u] = m;
       }
     }
-    if (lane == 0) a.ci_count[ci] = min(count, PGK_MAXJ);
-    if (__ballot(ovf) && lane == 0) atomicOr(a.overflow, 1);
-  } else if (ci <= a.ncl_max && lane == 0) {
-    a.ci_count[ci] = 0;   // slots past the real cluster count scan as empty
+  }
+  __syncthreads();
+  // one entry per half j-cluster with a listed pair: slots jj = 0..3 (mask
+  // bits 0..31) and jj = 4..7 (bits 32..63)
+  const int share = (ncand + PGK_FW - 1) / PGK_FW;
+  const int kb = min(wave * share, ncand), ke = min(kb + share, ncand);
+  int own = 0;
+  for (int k = kb; k < ke; k += 64) {
+    const uint64_t m = (k + lane < ke) ? s_mask[k + lane] : 0;
+    own += (int)(__popcll(__ballot((uint32_t)m != 0)) + __popcll(__ballot((m >> 32) != 0)));
+  }
+  // (the turn's counts of phase A are read: a barrier lies between)
+  if (lane == 0) s_cnt[0][wave] = own;
+  __syncthreads();
+  int at = 0, count = 0;
+#pragma unroll
+  for (int w2 = 0; w2 < PGK_FW; w2++) {
+    if (w2 < wave) at += s_cnt[0][w2];
+    count += s_cnt[0][w2];
+  }
+  for (int k = kb; k < ke; k += 64) {
+    const uint64_t m = (k + lane < ke) ? s_mask[k + lane] : 0;
+    const uint32_t m0 = (uint32_t)m, m1 = (uint32_t)(m >> 32);
+    const uint64_t b0 = __ballot(m0 != 0), b1 = __ballot(m1 != 0);
+    const int p0 = at + (int)(__popcll(b0 & below) + __popcll(b1 & below)), p1 = p0 + (m0 != 0);
+    const int cj2 = (k + lane < ke) ? 2 * cand[k + lane] : 0;
+    int32_t *tc = a.tmp_cj + (size_t)ci * PGK_MAXJ;
+    uint32_t *tm = a.tmp_mask + (size_t)ci * PGK_MAXJ;
+    if (m0 && p0 < PGK_MAXJ) {
+      tc[p0] = cj2;
+      tm[p0] = m0;
+    }
+    if (m1 && p1 < PGK_MAXJ) {
+      tc[p1] = cj2 + 1;
+      tm[p1] = m1;
+    }
+    at += (int)(__popcll(b0) + __popcll(b1));
+  }
+  if (wave == 0 && lane == 0) a.ci_count[ci] = min(count, PGK_MAXJ);
+  if (__ballot(ovf || count > PGK_MAXJ) && lane == 0) atomicOr(a.overflow, 1);
+}
+
+// Starts of the clusters' entries in the compact list, the starts of their
+// work items in the pair kernel's chunked form (chunk k of cluster ci holds
+// its entries 64 k .. 64 k + 63; at most 32 chunks, PGK_MAXJ = 2048 entries),
+// and the record the host waits for (in its own memory): clusters, overflow
+// flags (2: the list buffer is too small), entries, work items.  One block.
+__global__ __launch_bounds__(1024) void k_list_scan(const int32_t *__restrict__ d_ncl,
+                                                    const int32_t *__restrict__ ci_count,
+                                                    int32_t *__restrict__ ci_start,
+                                                    int32_t *__restrict__ wstart, int64_t cap,
+                                                    const int32_t *__restrict__ overflow,
+                                                    int32_t *__restrict__ meta) {
+  const int ncl = *d_ncl;
+  const uint64_t tot = block_scan(
+      ncl,
+      [&](int c) {
+        const int n = ci_count[c];
+        return ((uint64_t)((n + 63) / 64) << 32) | (uint32_t)n;
+      },
+      [&](int c, uint64_t at) {
+        ci_start[c] = (int32_t)(uint32_t)at;
+        wstart[c] = (int32_t)(at >> 32);
+      });
+  if (threadIdx.x == 0) {
+    const int32_t n = (int32_t)(uint32_t)tot, nw = (int32_t)(tot >> 32);
+    ci_start[ncl] = n;
+    wstart[ncl] = nw;
+    meta[0] = ncl;
+    meta[1] = *overflow | (n > cap ? 2 : 0);
+    meta[2] = n;
+    meta[3] = nw;
   }
 }
 
-// copy each cluster's entries to its place in the compact list; a list
-// buffer that is too small is reported (bit 2 of *overflow) and not written
-__global__ void k_compact_pairs(int ncl_max, const int32_t *__restrict__ ci_count,
-                                const int32_t *__restrict__ ci_start,
-                                const int32_t *__restrict__ tmp_cj,
-                                const uint32_t *__restrict__ tmp_mask,
-                                int32_t *__restrict__ cj, uint32_t *__restrict__ mask,
-                                int64_t cap, int32_t *__restrict__ overflow) {
+// copy each cluster's entries to its place in the compact list (a buffer that
+// is too small is not written past its end) and list its work items, coded
+// ci * 32 + chunk
+__global__ __launch_bounds__(256) void k_compact_pairs(
+    const int32_t *__restrict__ ncl, const int32_t *__restrict__ ci_start,
+    const int32_t *__restrict__ wstart, const int32_t *__restrict__ tmp_cj,
+    const uint32_t *__restrict__ tmp_mask, int32_t *__restrict__ cj, uint32_t *__restrict__ mask,
+    int64_t cap, int32_t *__restrict__ witem) {
   const int ci = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (ci >= ncl_max) return;
-  if (ci == 0 && lane == 0 && ci_start[ncl_max] > cap) atomicOr(overflow, 2);
-  const int n = ci_count[ci], s = ci_start[ci];
+  if (ci >= *ncl) return;
+  const int s = ci_start[ci], n = ci_start[ci + 1] - s;
   if ((int64_t)s + n > cap) return;
   for (int k = lane; k < n; k += 64) {
     cj[s + k] = tmp_cj[(size_t)ci * PGK_MAXJ + k];
     mask[s + k] = tmp_mask[(size_t)ci * PGK_MAXJ + k];
   }
-}
-
-// Work items of the pair kernel's chunked form: chunk k (entries 64 k ..
-// 64 k + 63 of its list) of cluster ci, coded ci * 32 + k (a cluster holds at
-// most PGK_MAXJ = 2048 entries, 32 chunks).
-__global__ void k_chunk_count(int ncl_max, const int32_t *__restrict__ ci_count,
-                              int32_t *__restrict__ wcount) {
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ci <= ncl_max) wcount[ci] = (ci < ncl_max) ? (ci_count[ci] + 63) / 64 : 0;
-}
-__global__ void k_chunk_fill(int ncl_max, const int32_t *__restrict__ wcount,
-                             const int32_t *__restrict__ wstart, int32_t *__restrict__ witem,
-                             int64_t cap) {
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ci >= ncl_max) return;
-  for (int k = 0; k < wcount[ci]; k++) {
-    const int64_t w = (int64_t)wstart[ci] + k;
-    if (w < cap) witem[w] = ci * 32 + k;
-  }
-}
-
-// cluster count, overflow flags, entry count and work-item count in one
-// record for the host
-__global__ void k_list_meta(const int32_t *__restrict__ ncl, const int32_t *__restrict__ ovf,
-                            const int32_t *__restrict__ tot, const int32_t *__restrict__ wtot,
-                            int32_t *__restrict__ meta) {
-  if (threadIdx.x == 0) {
-    meta[0] = *ncl;
-    meta[1] = *ovf;
-    meta[2] = *tot;
-    meta[3] = *wtot;
-  }
+  const int w = wstart[ci], nw = wstart[ci + 1] - w;
+  if (lane < nw) witem[w + lane] = ci * 32 + lane;
 }
 
 // number of listed atom pairs (bits set over all masks)
@@ -516,12 +621,9 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
   // kernels read the real count from the column scan, so nothing waits for
   // the host until the single read-back at the end
   const int ncl_max = n / PGK_CL + ncolumn + 1;
-  size_t need = 0, t1 = 0, t2 = 0;
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, t1, c->d_bin_count, c->d_bin_start,
+  size_t need = 0;
+  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, c->d_bin_count, c->d_bin_start,
                                              nbin + 1, st));
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, t2, c->d_bin_count, c->d_bin_start,
-                                             ncl_max + 1, st));
-  need = t1 > t2 ? t1 : t2;
   if (need > c->scan_tmp_bytes) {
     if (c->d_scan_tmp) (void)hipFree(c->d_scan_tmp);
     c->d_scan_tmp = nullptr;
@@ -537,7 +639,6 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
         (rc = dev_alloc(&c->d_tmp_mask, (size_t)ncl_max * PGK_MAXJ)) ||
         (rc = dev_alloc(&c->d_ci_count, (size_t)ncl_max + 4)) ||
         (rc = dev_alloc(&c->d_ci_start, (size_t)ncl_max + 4)) ||
-        (rc = dev_alloc(&c->d_wcount, (size_t)ncl_max + 4)) ||
         (rc = dev_alloc(&c->d_wstart, (size_t)ncl_max + 4)) ||
         (rc = dev_alloc(&c->d_witem, (size_t)ncl_max * (PGK_MAXJ / 64))) ||
         (rc = dev_alloc((int32_t **)&c->d_ct, ns)))
@@ -561,12 +662,8 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
     if ((rc = dev_alloc(&c->d_cj, cap)) || (rc = dev_alloc(&c->d_mask, cap))) return rc;
     c->cap_pair_cl = cap;
   }
-  if (!c->d_list_meta) {
-    HIP_CHECK(hipMalloc(&c->d_list_meta, 4 * sizeof(int32_t)));
-    HIP_CHECK(hipHostMalloc(&c->h_list_meta, 4 * sizeof(int32_t)));
-  }
+  if (!c->h_list_meta) HIP_CHECK(hipHostMalloc(&c->h_list_meta, 4 * sizeof(int32_t)));
   HIP_CHECK(hipMemsetAsync(c->d_bin_count, 0, sizeof(int32_t) * (nbin + 1), st));
-  HIP_CHECK(hipMemsetAsync(c->d_overflow, 0, sizeof(int32_t), st));
   k_bin_atoms<<<pgk_grid_blocks(n, 256), 256, 0, st>>>(c->d_pos, n, g, c->d_bin_count,
                                                         c->d_atom_bin, c->d_atom_slot);
   HIP_CHECK(hipGetLastError());
@@ -576,18 +673,12 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
   k_scatter<<<pgk_grid_blocks(n, 256), 256, 0, st>>>(n, c->d_atom_bin, c->d_atom_slot,
                                                       c->d_bin_start, c->d_sorted);
   k_sort_bins<<<pgk_grid_blocks(nbin, 256), 256, 0, st>>>(nbin, c->d_bin_start, c->d_sorted);
-  k_col_counts<<<pgk_grid_blocks(ncolumn, 256), 256, 0, st>>>(ncolumn, g.nzb, c->d_bin_start,
-                                                              c->d_col_ncl);
-  HIP_CHECK(hipMemsetAsync(c->d_col_ncl + ncolumn, 0, sizeof(int32_t), st));
-  tb = c->scan_tmp_bytes;
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(c->d_scan_tmp, tb, c->d_col_ncl, c->d_col_clstart,
-                                             ncolumn + 1, st));
+  k_col_scan<<<1, 1024, 0, st>>>(ncolumn, g.nzb, c->d_bin_start, c->d_col_ncl, c->d_col_clstart,
+                                 c->d_overflow);
   const int32_t *d_ncl = c->d_col_clstart + ncolumn;
-  k_fill_clusters<<<ncolumn, 64, 0, st>>>(g.nzb, c->d_bin_start, c->d_sorted, c->d_col_ncl,
-                                          c->d_col_clstart, c->d_cl_atom, c->d_cl_col,
-                                          c->d_slot_of);
-  k_bbox<<<pgk_grid_blocks(ncl_max, 128), 128, 0, st>>>(d_ncl, c->d_pos, c->d_cl_atom, g,
-                                                        c->d_bbox, c->d_posc);
+  k_fill_clusters<<<ncolumn, 64, 0, st>>>(g, c->d_bin_start, c->d_sorted, c->d_col_ncl,
+                                          c->d_col_clstart, c->d_pos, c->d_cl_atom, c->d_cl_col,
+                                          c->d_slot_of, c->d_bbox, c->d_posc);
   HIP_CHECK(hipGetLastError());
 
   ListArgs a;
@@ -605,7 +696,6 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
   a.ci_count = c->d_ci_count;
   a.overflow = c->d_overflow;
   a.ncolumn = ncolumn;
-  a.ncl_max = ncl_max;
   for (int d = 0; d < 2; d++) {
     a.ncol[d] = g.ncol[d];
     a.rng[d] = (int)ceil(rcut_book / g.colw[d]);
@@ -617,35 +707,23 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
     a.Lf[d] = (float)g.L[d];
   }
   a.sqcut = rcut_book * rcut_book;
+  const bool wide = std::min(g.L[0], std::min(g.L[1], g.L[2])) > 2.0001 * rcut_book;
   float rf = (float)rcut_book + 1e-3f;
   a.rcbf2 = rf * rf;
   // reach plus one z bin (cluster z bounds are ordered only up to a bin) and
   // a margin for the bounding-box padding and float rounding
   a.zwin = rf + (float)g.zbw + 0.01f;
-  // blocks cover ci = 0 .. ncl_max so that the count past the end is cleared
-  if ((int64_t)ncl_max < c->pair_chunk_below)
-    k_find_pairs<1><<<ncl_max + 1, 64, 0, st>>>(a);
-  else
-    k_find_pairs<4><<<(ncl_max + 1 + 3) / 4, 256, 0, st>>>(a);
+  if (wide) k_find_pairs<true><<<ncl_max, 64 * PGK_FW, 0, st>>>(a);
+  else k_find_pairs<false><<<ncl_max, 64 * PGK_FW, 0, st>>>(a);
+  k_list_scan<<<1, 1024, 0, st>>>(d_ncl, c->d_ci_count, c->d_ci_start, c->d_wstart,
+                                  c->cap_pair_cl, c->d_overflow, c->h_list_meta);
+  auto compact = [&] {
+    k_compact_pairs<<<(ncl_max + 3) / 4, 256, 0, st>>>(d_ncl, c->d_ci_start, c->d_wstart,
+                                                       c->d_tmp_cj, c->d_tmp_mask, c->d_cj,
+                                                       c->d_mask, c->cap_pair_cl, c->d_witem);
+  };
+  compact();
   HIP_CHECK(hipGetLastError());
-  tb = c->scan_tmp_bytes;
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(c->d_scan_tmp, tb, c->d_ci_count, c->d_ci_start,
-                                             ncl_max + 1, st));
-  k_compact_pairs<<<(ncl_max + 3) / 4, 256, 0, st>>>(ncl_max, c->d_ci_count, c->d_ci_start,
-                                                     c->d_tmp_cj, c->d_tmp_mask, c->d_cj,
-                                                     c->d_mask, c->cap_pair_cl, c->d_overflow);
-  k_chunk_count<<<pgk_grid_blocks(ncl_max + 1, 256), 256, 0, st>>>(ncl_max, c->d_ci_count,
-                                                                   c->d_wcount);
-  tb = c->scan_tmp_bytes;
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(c->d_scan_tmp, tb, c->d_wcount, c->d_wstart,
-                                             ncl_max + 1, st));
-  k_chunk_fill<<<pgk_grid_blocks(ncl_max, 256), 256, 0, st>>>(
-      ncl_max, c->d_wcount, c->d_wstart, c->d_witem, (int64_t)ncl_max * (PGK_MAXJ / 64));
-  k_list_meta<<<1, 64, 0, st>>>(d_ncl, c->d_overflow, c->d_ci_start + ncl_max,
-                                c->d_wstart + ncl_max, c->d_list_meta);
-  HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(c->h_list_meta, c->d_list_meta, 4 * sizeof(int32_t),
-                           hipMemcpyDeviceToHost, st));
   HIP_CHECK(hipStreamSynchronize(st));
   const int32_t ncl = c->h_list_meta[0], ovf = c->h_list_meta[1], tot = c->h_list_meta[2];
   c->nwi = c->h_list_meta[3];
@@ -658,9 +736,7 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
     const int64_t cap = (int64_t)(tot * 1.25) + 1024;
     if ((rc = dev_alloc(&c->d_cj, cap)) || (rc = dev_alloc(&c->d_mask, cap))) return rc;
     c->cap_pair_cl = cap;
-    k_compact_pairs<<<(ncl_max + 3) / 4, 256, 0, st>>>(ncl_max, c->d_ci_count, c->d_ci_start,
-                                                       c->d_tmp_cj, c->d_tmp_mask, c->d_cj,
-                                                       c->d_mask, c->cap_pair_cl, c->d_overflow);
+    compact();
     HIP_CHECK(hipGetLastError());
   }
   c->ncl = ncl;
@@ -678,7 +754,7 @@ int pgk_list_build(pgk_ctx *c, double rcut_book) {
 int pgk_list_count_pairs(pgk_ctx *c) {
   if (c->npairs >= 0) return PGK_OK;
   hipStream_t st = c->stream;
-  unsigned long long *d_np = reinterpret_cast<unsigned long long *>(c->d_list_meta);
+  unsigned long long *d_np = reinterpret_cast<unsigned long long *>(c->d_overflow + 2);
   HIP_CHECK(hipMemsetAsync(d_np, 0, sizeof(unsigned long long), st));
   if (c->npair_cl > 0) {
     const int nb = (int)std::min<int64_t>(1024, (c->npair_cl + 255) / 256);

@@ -917,8 +917,7 @@ int pgk_destroy(pgk_ctx *c) {
                   c->d_rb, c->d_p14, c->d_p14f, c->d_bpar, c->d_bin_count, c->d_bin_start,
                   c->d_atom_bin, c->d_atom_slot, c->d_sorted, c->d_col_ncl, c->d_col_clstart,
                   c->d_cl_atom, c->d_cl_col, c->d_slot_of, c->d_bbox, c->d_posc, c->d_tmp_cj,
-                  c->d_list_meta,
-                  c->d_tmp_mask, c->d_wcount, c->d_wstart, c->d_witem, c->d_ci_count, c->d_ci_start, c->d_cj, c->d_mask,
+                  c->d_tmp_mask, c->d_wstart, c->d_witem, c->d_ci_count, c->d_ci_start, c->d_cj, c->d_mask,
                   c->d_overflow, c->d_scan_tmp, c->d_xq, c->d_ct, c->d_fcl, c->d_fat,
                   c->d_fcl_c, c->d_fat_c, c->d_force, c->d_fvc, c->d_fvl, c->d_red, c->d_sum,
                   c->d_grid, c->d_pgrid, c->d_cgrid, c->d_tw, c->d_twf, c->d_theta, c->d_tile,

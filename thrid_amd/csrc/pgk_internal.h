@@ -189,7 +189,7 @@ struct pgk_ctx {
   int32_t *d_ci_count = nullptr, *d_ci_start = nullptr;
   // the pair kernel's work items in its chunked form (64 list entries of one
   // cluster each, coded cluster * 32 + chunk) and their count
-  int32_t *d_wcount = nullptr, *d_wstart = nullptr, *d_witem = nullptr;
+  int32_t *d_wstart = nullptr, *d_witem = nullptr;
   int nwi = 0;
   int64_t pair_chunk_below = PGK_TUNE_DEFAULT_CHUNK_BELOW;   // chunked form below this ncl
   int pair_cap_default = 2;        // pair blocks per CU beside the chain (0: no cap)
@@ -197,8 +197,8 @@ struct pgk_ctx {
   int32_t *d_cj = nullptr;         // entries: half-cluster index 2 cj + h
   uint32_t *d_mask = nullptr;      // entries: bit ii + 8 jq for i-slot ii, j-slot 4 h + jq
   int64_t npair_cl = 0, cap_pair_cl = 0;
-  int32_t *d_list_meta = nullptr;  // cluster count, overflow flags, entry count
-  int32_t *h_list_meta = nullptr;  // pinned copy read once per rebuild
+  int32_t *h_list_meta = nullptr;  // cluster count, overflow flags, entry and work-item
+                                   // counts: pinned, written by the rebuild's scan
   int64_t npairs = 0;              // atom pairs in the list
   int32_t *d_overflow = nullptr;
   void *d_scan_tmp = nullptr;
