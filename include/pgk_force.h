@@ -580,7 +580,8 @@ int pgk_profile_stages(pgk_ctx *ctx, uint32_t mask);
  *     PGK_TUNE_DEFAULT_CHUNK_BELOW, the crossover thrid_amd/autotune.py
  *     measured (thrid_amd/tuning.json).
  *   PGK_TUNE_PME_OVERLAP: 1 (default) runs the reciprocal chain on a second
- *     stream beside the pair kernel when both are due, 0 one after the other.
+ *     stream beside the pair kernel when both are due (in dynamics, and the
+ *     system is large enough to gain), 0 one after the other.
  *   PGK_TUNE_PAIR_CAP_BLOCKS: pair blocks per CU while the chain runs beside
  *     them (default 2; 0 no cap); the chunked form keeps 3 unless 0.        */
 enum { PGK_TUNE_PAIR_CHUNK_BELOW = 1, PGK_TUNE_PME_OVERLAP = 2, PGK_TUNE_PAIR_CAP_BLOCKS = 3 };

@@ -317,7 +317,20 @@ int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom
   // beside it (timing any stage but the pair kernel keeps them one after
   // the other)
   const bool timed_other = c->prof && (c->prof_mask & ~(1u << PGK_PROF_PAIRS)) != 0;
-  const bool overlap = do_pair && do_ewk && !hf && !timed_other && c->pme_overlap;
+  // A step queued ahead (no wait) pays about 12 us for the fork and the join,
+  // which the shorter side of a small system does not earn back.  us per step,
+  // beside / one after the other, by list entries + grid points: water, mixed
+  // 20 k 102/95, 177 k 114/109, 278 k 118/112, 436 k 138/132, 548 k 137/137,
+  // 704 k 129/144; FP64 278 k 122/117, 436 k 147/145, 548 k 142/156.  With
+  // bonds and angles beside the chain as well the line lies lower (FP64 slab
+  // of 378 k: 140/144; with them in RESPA's short calls 349/339).  A caller that waits is bound by the host's launches, which two queues take
+  // side by side (648 atoms: 149 us against 154).
+  const bool bonded = (c->nbond_act > 0 && m->bond == mts_flag) ||
+                      (c->nangl_act > 0 && m->angl == mts_flag);
+  const int64_t work = c->npair_cl + (int64_t)c->nfft[0] * c->nfft[1] * c->nfft[2];
+  const bool small = !wait && work < (bonded ? 300000 : 450000);
+  const bool overlap =
+      do_pair && do_ewk && !hf && !timed_other && c->pme_overlap && !small;
   // beside the chain the excluded-pair correction goes to the shorter stream:
   // the pair kernel's where the chain outlasts the pair and bonded kernels
   // (small systems in the chunked form; the FP64 form, whose chain runs in
