@@ -1708,6 +1708,7 @@ struct MdRunner {
   bool graphs;
   hipGraphExec_t gexec = nullptr;
   bool primed = false;
+  bool opened = false;   // the chain's opening call of the next step is done
   MdRunner(pgk_ctx *ctx, bool use_graphs) : c(ctx), graphs(use_graphs) {}
   ~MdRunner() { drop(); }
   void drop() {
@@ -1725,16 +1726,20 @@ struct MdRunner {
   // changed the others, and a registration may have moved atoms between the
   // sets, so the opening call takes fresh records of the chain's atoms.
   int nhc_open() {
-    int r;
     if (!c->md_nhc_m) return PGK_OK;
-    if (c->md_lt_nreg && (r = pgk_md_ke(c, c->d_md_kenhc, true))) return r;
-    return pgk_md_nhc_half(c);
+    if (opened) {
+      opened = false;
+      return PGK_OK;
+    }
+    return c->md_lt_nreg ? pgk_md_ke_nhc(c, 1) : pgk_md_nhc_half(c);
   }
-  int nhc_close() {
-    int r;
+  // A step that samples nothing is followed by another of this run (the last
+  // one samples), so its closing launch makes that step's opening call as
+  // well; a replayed graph holds whole steps and does not.
+  int nhc_close(bool ene) {
     if (!c->md_nhc_m) return PGK_OK;
-    if ((r = pgk_md_ke(c, c->d_md_kenhc, true))) return r;
-    return pgk_md_nhc_half(c);
+    opened = !ene && !graphs && !c->md_lt_nreg;
+    return pgk_md_ke_nhc(c, opened ? 2 : 1);
   }
   int eager(bool ene) {
     int r;
@@ -1744,7 +1749,7 @@ struct MdRunner {
                           nullptr, nullptr, false, false, ene)))
       return r;
     if ((r = pgk_md_kick(c, c->d_force, c->md_dt, nullptr, 0.0))) return r;
-    return nhc_close();
+    return nhc_close(ene);
   }
   // Region Langevin thermostat: its first half opens the step, before the
   // first half kick; at the close the atoms are registered at the new
@@ -1856,7 +1861,7 @@ struct MdRunner {
     if ((r = run_calforce(c, PGK_MTS_LONG, &kMdMts, 0, false, c->d_force, nullptr, nullptr,
                           nullptr, nullptr, false, false, ene)))
       return r;
-    if ((r = pgk_md_kick(c, c->d_force, c->md_dt, nullptr, 0.0)) || (r = nhc_close()) ||
+    if ((r = pgk_md_kick(c, c->d_force, c->md_dt, nullptr, 0.0)) || (r = nhc_close(ene)) ||
         (r = lt_close()))
       return r;
     if (plain) primed = true;
@@ -2032,7 +2037,7 @@ int pgk_md_nhc(pgk_ctx *c, const pgk_nhc_desc *nhc) {
   }
   // kT in eref, masses in eref fs^2 (prepmd.F90:515-518)
   const double gkt = 1.380649e-23 / 6.9511042e-21 * nhc->temperature;
-  std::vector<double> st((size_t)3 * m + 2, 0.0);
+  std::vector<double> st((size_t)3 * m + 3, 0.0);
   for (int i = 0; i < m; i++) {
     st[i] = nhc->xlogs ? nhc->xlogs[i] : 0.0;
     st[m + i] = nhc->vlogs ? nhc->vlogs[i] : 0.0;
