@@ -1257,9 +1257,9 @@ static int hf_setup(pgk_ctx *c, const pgk_hf_desc *hf, bool flux, const char *wh
     const size_t jcol_b = sizeof(double) * PGK_NHF * (size_t)nreg * 3;
     const size_t nblk = (size_t)pgk_grid_blocks(std::max<int64_t>(pgk_pair_waves(c), 1), 4);
     // bulk: 12 flux sums and 12 transport sums per block; volume: 4 classes of
-    // two words per region and a flag (k_hf_vol.hip)
+    // three words per region, and the velocities' exponents (k_hf_vol.hip)
     const bool bulk = hf->mode == PGK_HF_BULK;
-    const size_t jpart_b = sizeof(double) * (bulk ? nblk * 24 : 8 * (size_t)nreg + 1);
+    const size_t jpart_b = sizeof(double) * (bulk ? nblk * 24 : 12 * (size_t)nreg + 2);
     if ((rc = grow_dev((void **)&c->d_hj_jcol, &c->hj_jcol_cap, jcol_b)) ||
         (rc = grow_dev((void **)&c->d_hj_jpart, &c->hj_jpart_cap, jpart_b)))
       return rc;

@@ -60,7 +60,7 @@ void pgk_set_error(const std::string &msg);
 // eref / (amu A^2 fs^-2): a = F/m * PGK_MD_CONV, KE = m v^2 / 2 / PGK_MD_CONV
 #define PGK_MD_CONV (6.9511042e-21 / 1.66053907e-17)
 
-// volume regions of the flux form: the regions' sums keep [17][nreg] doubles of
+// volume regions of the flux form: the regions' sums keep [16][nreg] doubles of
 // LDS per wave
 #define PGK_HEATF_MAXREG 1024
 
@@ -96,7 +96,8 @@ struct HfDev {
   int direct_ok = 0, direct_tr = 0;
   int vol_pairs = 0;                           // volume mode: the pair pass has run
   double *jcol = nullptr;   // [PGK_NHF][nreg][3] sums, heat-flux accumulator type (int64 fixed point in the mixed form)
-  // bulk pair pass: per-block records; volume: sums of the pairs on a plane
+  // bulk pair pass: per-block records; volume: the pairs weighed region by
+  // region and the velocities' exponents (k_hf_vol.hip)
   double *jpart = nullptr;
 };
 
