@@ -26,12 +26,13 @@
 // (With FP64 sums per atom instead the pair pass took 4.6 ms there, and 98 us
 // against 117 on an 18,000-atom slab in FP64.)
 //
-// Two kinds of pair are weighed region by region instead, into jpart:
+// Three kinds of pair are weighed region by region instead, into jpart:
 // - a first atom whose centre lies exactly on a region's plane, with the
 //   second on the far side of it: there the reference's rule counts the whole
 //   segment (kTypPlane; the atoms' shares count the rest);
 // - a share of 2^24 units and more, infinite or NaN (atoms on top of each
-//   other): it reaches the regions its segment meets and no other.
+//   other): it reaches the regions its segment meets and no other;
+// - every pair, if a region's bounds are the wrong way round (h.reversed).
 //
 // Energies per slot of the cluster list: FP64 in the FP64 and FP32 forms, 2^-32
 // fixed point like the forces in the mixed form.
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(256) void k_hf_pairs_vol(HfVolArgs p, HfDev h,
             fv = (R)12 * ep * (t12 - t6) * rinv2;
           }
           double sc = seg ? (double)fc * rw : 0.0, sv = seg ? (double)fv * rw : 0.0;
-          const bool whole = !(fabs(sc) < kVolMax && fabs(sv) < kVolMax);
+          const bool whole = h.reversed || !(fabs(sc) < kVolMax && fabs(sv) < kVolMax);
           if (__builtin_expect(whole || (plane && dz != 0.0), 0)) {
             vol_regions(h, whole, same ? 0 : 2, vi.w, d.vj.w, sc, sv);
             if (whole) sc = sv = 0.0;

@@ -1231,6 +1231,9 @@ static int hf_setup(pgk_ctx *c, const pgk_hf_desc *hf, bool flux, const char *wh
     for (int r = 0; tiled && r < nreg; r++)
       tiled = hf->z1[r] < hf->z2[r] && (r + 1 == nreg || hf->z2[r] == hf->z1[r + 1]);
     h.tiled = tiled ? 1 : 0;
+    bool rev = false;
+    for (int r = 0; r < nreg; r++) rev = rev || !(hf->z1[r] <= hf->z2[r]);
+    h.reversed = rev ? 1 : 0;
   }
   h.hftyp = c->d_hf_typ;
   h.molid = c->d_molid;

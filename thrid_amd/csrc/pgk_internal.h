@@ -75,7 +75,8 @@ struct HfDev {
   // tiled = 1 when moreover each region ends exactly where the next begins
   // (z2[r] == z1[r + 1]) and z1 increases strictly: a segment's regions
   // strictly between its end regions then take its full width
-  int ubin = 0, tiled = 0;
+  // reversed = 1: not every region has z1 <= z2
+  int ubin = 0, tiled = 0, reversed = 0;
   double ubz0 = 0.0, ubw = 1.0, ubwi = 1.0;
   const int32_t *hftyp = nullptr;              // [natom] 1 = ATOM, 2 = MOLE
   const int32_t *molid = nullptr;              // [natom] 1-based
