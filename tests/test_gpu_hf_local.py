@@ -101,6 +101,19 @@ def test_bad_pair_stays_in_its_region(prec, tol):
     assert not abs(got[bad, row, 2]) < 1e6 * np.max(np.abs(ref[rest, row, 2]))
 
 
+def test_close_pair_without_lj_mixed():
+    """An H atom (no LJ) 5e-4 A from an O: the LJ terms of FP32 overflow and
+    count nothing."""
+    s, bad = _close_pair(small_slab(), "HB", "OB", 5e-4)
+    z = np.arange(61.0)
+    vel = md.maxwell_boltzmann(s, 300.0, seed=44)
+    got, ref, _ = _calls(s, "mixed", z[:-1], z[1:], vel)
+    for row in (abi.HFJ_VIRI + abi.HF_NAMES.index("vdw"),
+                abi.HFJ_POT + abi.HF_NAMES.index("vdw")):
+        d = np.abs(got[:, row, 2] - ref[:, row, 2])
+        assert np.max(d) < 1e-7 * np.max(np.abs(ref[:, row, 2]))
+
+
 def _weight(z1, z2, ci, cj):
     """calvirihf's weight of a region for the segment cj -> ci."""
     ri1, rj1, ri2, rj2 = ci - z1, cj - z1, ci - z2, cj - z2
