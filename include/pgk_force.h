@@ -580,8 +580,11 @@ int pgk_profile_stages(pgk_ctx *ctx, uint32_t mask);
  *     PGK_TUNE_DEFAULT_CHUNK_BELOW, the crossover thrid_amd/autotune.py
  *     measured (thrid_amd/tuning.json).
  *   PGK_TUNE_PME_OVERLAP: 1 (default) runs the reciprocal chain on a second
- *     stream beside the pair kernel when both are due (in dynamics, and the
- *     system is large enough to gain), 0 one after the other.
+ *     stream beside the pair kernel when both are due, 0 one after the other.
+ *     Until it is set, the steps of a trajectory under RESPA or without bonded
+ *     terms run them one after the other in systems too small to gain (list
+ *     entries and grid points together below 450000); setting 1 runs them side
+ *     by side there too.
  *   PGK_TUNE_PAIR_CAP_BLOCKS: pair blocks per CU while the chain runs beside
  *     them (default 2; 0 no cap); the chunked form keeps 3 unless 0.        */
 enum { PGK_TUNE_PAIR_CHUNK_BELOW = 1, PGK_TUNE_PME_OVERLAP = 2, PGK_TUNE_PAIR_CAP_BLOCKS = 3 };

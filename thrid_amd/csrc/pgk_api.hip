@@ -254,7 +254,7 @@ int finalize_energies(pgk_ctx *c, double *ene, double *virt);
 
 int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom, bool split,
                  double *d_force_out, double *d_fvc, double *d_fvl, double *ene, double *virt,
-                 bool hf = false, bool wait = true, bool energies = true) {
+                 bool hf = false, bool wait = true, bool energies = true, bool step = false) {
   if (!c->have_pos) {
     pgk_set_error("pgk_calforce: positions not set");
     return PGK_ESTATE;
@@ -314,23 +314,14 @@ int run_calforce(pgk_ctx *c, int32_t mts_flag, const pgk_mts *m, int32_t preatom
   // The reciprocal chain (spread, FFT, gather) and the pair kernel read the
   // same positions and write different accumulators: with both due, the
   // chain goes to the second stream and the pair and bonded kernels run
-  // beside it (timing any stage but the pair kernel keeps them one after
-  // the other)
+  // beside it, where that pays (pgk_pme_beside; timing any stage but the
+  // pair kernel keeps them one after the other)
   const bool timed_other = c->prof && (c->prof_mask & ~(1u << PGK_PROF_PAIRS)) != 0;
-  // A step queued ahead (no wait) pays about 12 us for the fork and the join,
-  // which the shorter side of a small system does not earn back.  us per step,
-  // beside / one after the other, by list entries + grid points: water, mixed
-  // 20 k 102/95, 177 k 114/109, 278 k 118/112, 436 k 138/132, 548 k 137/137,
-  // 704 k 129/144; FP64 278 k 122/117, 436 k 147/145, 548 k 142/156.  With
-  // bonds and angles beside the chain as well the line lies lower (FP64 slab
-  // of 378 k: 140/144; with them in RESPA's short calls 349/339).  A caller that waits is bound by the host's launches, which two queues take
-  // side by side (648 atoms: 149 us against 154).
-  const bool bonded = (c->nbond_act > 0 && m->bond == mts_flag) ||
-                      (c->nangl_act > 0 && m->angl == mts_flag);
-  const int64_t work = c->npair_cl + (int64_t)c->nfft[0] * c->nfft[1] * c->nfft[2];
-  const bool small = !wait && work < (bonded ? 300000 : 450000);
   const bool overlap =
-      do_pair && do_ewk && !hf && !timed_other && c->pme_overlap && !small;
+      do_pair && do_ewk && !hf && !timed_other &&
+      pgk_pme_beside(c->pme_overlap, c->pme_overlap_chosen, step,
+                     pgk_bonded_due(c, m, mts_flag) && c->md_nshort <= 1,
+                     c->npair_cl + (int64_t)c->nfft[0] * c->nfft[1] * c->nfft[2]);
   // beside the chain the excluded-pair correction goes to the shorter stream:
   // the pair kernel's where the chain outlasts the pair and bonded kernels
   // (small systems in the chunked form; the FP64 form, whose chain runs in
@@ -1749,7 +1740,7 @@ struct MdRunner {
     if ((r = nhc_open()) || (r = pgk_md_kick_drift(c, c->d_force, c->md_dt, nullptr, 0.0)))
       return r;
     if ((r = run_calforce(c, PGK_MTS_LONG, &kMdMts, 0, false, c->d_force, nullptr, nullptr,
-                          nullptr, nullptr, false, false, ene)))
+                          nullptr, nullptr, false, false, ene, true)))
       return r;
     if ((r = pgk_md_kick(c, c->d_force, c->md_dt, nullptr, 0.0))) return r;
     return nhc_close(ene);
@@ -1772,7 +1763,7 @@ struct MdRunner {
   int short_forces(bool ene) {
     if (!ene)
       return run_calforce(c, PGK_MTS_SHORT, &c->md_mts, 0, false, c->d_md_fshort, nullptr,
-                          nullptr, nullptr, nullptr, false, false, false);
+                          nullptr, nullptr, nullptr, false, false, false, true);
     for (double &e : c->md_e_short) e = 0.0;
     return run_calforce(c, PGK_MTS_SHORT, &c->md_mts, 0, false, c->d_md_fshort, nullptr,
                         nullptr, c->md_e_short, nullptr, false, true, true);
@@ -1797,7 +1788,7 @@ struct MdRunner {
       }
       if ((r = short_forces(ene && last))) return r;
       if (last && (r = run_calforce(c, PGK_MTS_LONG, &c->md_mts, 0, false, c->d_force, nullptr,
-                                    nullptr, nullptr, nullptr, false, false, ene)))
+                                    nullptr, nullptr, nullptr, false, false, ene, true)))
         return r;
       if ((r = pgk_md_kick(c, c->d_md_fshort, dts, last ? c->d_force : nullptr, c->md_dt)))
         return r;
@@ -1819,10 +1810,10 @@ struct MdRunner {
     if (respa()) {
       if ((r = short_forces(true))) return r;
       return run_calforce(c, PGK_MTS_LONG, &c->md_mts, 0, false, c->d_force, nullptr, nullptr,
-                          nullptr, nullptr, false, false);
+                          nullptr, nullptr, false, false, true, true);
     }
     return run_calforce(c, PGK_MTS_LONG, &kMdMts, 0, false, c->d_force, nullptr, nullptr,
-                        nullptr, nullptr, false, false);
+                        nullptr, nullptr, false, false, true, true);
   }
   int step(bool rebuild, bool ene, double rcut_book) {
     int r;
@@ -1862,7 +1853,7 @@ struct MdRunner {
       if ((r = pgk_build_list(c, rcut_book))) return r;
     }
     if ((r = run_calforce(c, PGK_MTS_LONG, &kMdMts, 0, false, c->d_force, nullptr, nullptr,
-                          nullptr, nullptr, false, false, ene)))
+                          nullptr, nullptr, false, false, ene, true)))
       return r;
     if ((r = pgk_md_kick(c, c->d_force, c->md_dt, nullptr, 0.0)) || (r = nhc_close(ene)) ||
         (r = lt_close()))
@@ -2378,6 +2369,7 @@ int pgk_tune(pgk_ctx *c, int32_t knob, int64_t value) {
     case PGK_TUNE_PME_OVERLAP:
       if (value != 0 && value != 1) break;
       c->pme_overlap = value != 0;
+      c->pme_overlap_chosen = true;
       return PGK_OK;
     case PGK_TUNE_PAIR_CAP_BLOCKS:
       if (value < 0 || value > 16) break;

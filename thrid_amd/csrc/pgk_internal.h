@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "pgk_force.h"
+#include "pgk_rules.h"
 
 #define PGK_CL 8             // atoms per cluster
 #define PGK_MAXJ 2048        // max candidates / half-cluster entries per i-cluster
@@ -115,6 +116,7 @@ struct pgk_ctx {
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool pme_overlap = true;
+  bool pme_overlap_chosen = false;   // set by pgk_tune: whatever the system's size
   int pair_cap_blocks = 0;         // >0: pair blocks per CU while the chain runs beside
   int lds_per_cu = 0;              // bytes of LDS per CU
   int precision = PGK_PREC_FP64;
@@ -445,6 +447,13 @@ static inline bool pgk_pair_chunked(const pgk_ctx *c) {
 static inline bool pgk_has_bonded(const pgk_ctx *c) {
   return c->nbond_act > 0 || c->nangl_act > 0 || !c->tors_type.empty() || !c->rb_type.empty() ||
          c->n14 > 0;
+}
+
+// bonded terms due in a call at this level
+static inline bool pgk_bonded_due(const pgk_ctx *c, const pgk_mts *m, int flag) {
+  return (c->nbond_act > 0 && m->bond == flag) || (c->nangl_act > 0 && m->angl == flag) ||
+         (!c->tors_type.empty() && m->tors == flag) ||
+         (!c->rb_type.empty() && m->torsrb == flag) || (c->n14 > 0 && m->nonb14 == flag);
 }
 
 // waves of a pass over the current list in the form pgk_pair_chunked picks
