@@ -357,11 +357,15 @@ __device__ __forceinline__ void atom_frac_t(const double *pos, int i, const PmeG
 // no scan and no second pass over the slots.  Those were two launches of 4-5
 // us in a chain that bounds small systems: 24,000 atoms in FP32 155 -> 146 us
 // per step, an 18,000-atom slab 169 -> 163, 5,079 atoms with heat flux 190 ->
-// 185.  An atom moves less than the list's margin between builds, under one
-// tile, so few slots overflow; each costs every tile one look.
+// 185.  Between the builds of a trajectory atoms move by a part of the list's
+// margin and few slots overflow.  Each costs every tile one look (24,000 atoms
+// squeezed to an eighth of the box behind a list's back: spreading 113 us
+// against 33), so a call that finds more than bin_extra_max sets *full, in the
+// host's memory, and the next preparation takes new starts.
 struct BinRef {
-  int32_t *count, *start, *items, *extra, *extra_items;
+  int32_t *count, *start, *items, *extra, *extra_items, *full;
 };
+__device__ __forceinline__ int bin_extra_max(int nitem) { return 64 + nitem / 512; }
 
 // Per-slot preparation ahead of the force kernels, in the list's spatial order
 // (order[k] = atom, or -1 for padding; identity without a list):
@@ -491,7 +495,10 @@ __global__ __launch_bounds__(256) void k_gather_t(int nitem, const int32_t *__re
   const int t = xcd_block() * blockDim.x + threadIdx.x;
   // the spreading is done: the bins start empty at the next call
   for (int z = t; z < ntile; z += gridDim.x * blockDim.x) bin.count[z] = 0;
-  if (t == 0) bin.extra[0] = 0;
+  if (t == 0) {
+    if (bin.extra[0] > bin_extra_max(nitem)) *bin.full = 1;
+    bin.extra[0] = 0;
+  }
   const int k = t >> 2, sub = t & 3;
   // whole groups of four lanes leave together, so the shuffles below see
   // their partners
@@ -1680,6 +1687,7 @@ static int pme_layout(pgk_ctx *c, size_t rsize, PmeLayout *L) {
   L->bin.start = L->bin.extra + 1;
   L->bin.extra_items = L->bin.start + tg.ntile + 1;
   L->bin.items = L->bin.extra_items + nitem;
+  L->bin.full = c->h_bins_full;
   return PGK_OK;
 }
 
@@ -1692,8 +1700,18 @@ int launch_prep(pgk_ctx *c) {
   if (rc) return rc;
   const int gb = pgk_grid_blocks(L.nitem, 256);
   // the bins' starts follow the list: a rebuild changes the slots and comes
-  // where the atoms have moved; without a list (charges alone) nothing bounds
-  // the motion between calls and each call takes new ones
+  // where the atoms have moved; without a list (charges alone) each call takes
+  // new ones.  Atoms that moved far without a rebuild are noticed a call later
+  // (not in a step being captured: its replays would take new ones each time)
+  volatile int32_t *full = L.bin.full;
+  if (*full) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(c->stream, &cap));
+    if (cap == hipStreamCaptureStatusNone) {
+      *full = 0;
+      c->tile_serial = -1;
+    }
+  }
   if (!L.order || c->tile_serial != c->list_serial || c->tile_nitem != L.nitem) {
     k_bin_count<<<gb, 256, 0, c->stream>>>(L.nitem, L.order, c->d_pos, L.g, L.tg, L.bin.count);
     HIP_CHECK(hipGetLastError());

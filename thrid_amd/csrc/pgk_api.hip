@@ -900,6 +900,10 @@ int pgk_create(const pgk_system_desc *d, int32_t precision, pgk_ctx **out) {
   if (he == hipSuccess) he = hipMalloc(&c->d_cgrid, Hc * csz);
   if (he == hipSuccess) he = hipMalloc((void **)&c->d_sum, sizeof(double) * 1024);
   if (he == hipSuccess) he = hipHostMalloc((void **)&c->h_sum, sizeof(double) * 1024);
+  if (he == hipSuccess) {
+    c->h_bins_full = reinterpret_cast<int32_t *>(c->h_sum + 1023);
+    *c->h_bins_full = 0;
+  }
   if (he != hipSuccess) {
     pgk_set_error(std::string("pgk_create: device allocation failed: ") + hipGetErrorString(he));
     pgk_destroy(c);

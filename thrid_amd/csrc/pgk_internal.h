@@ -234,6 +234,7 @@ struct pgk_ctx {
   size_t tile_bytes = 0;
   int tile_ntile = 0, tile_nitem = 0;
   int64_t tile_serial = -1;        // the list build the bins' starts are of
+  int32_t *h_bins_full = nullptr;  // in h_sum: set by a call whose bins overflowed
   double *d_tw = nullptr;          // twiddles: 3 dims, each n complex (FP64)
   float *d_twf = nullptr;
   int tw_off[3] = {0, 0, 0};
