@@ -1208,59 +1208,23 @@ struct ConvArgs {
   int ifnetq;
 };
 
-// Influence function of mode (h, k2, k3) (scalar_sum, fft_pme.F90:544-690):
-// returns eterm (0 outside |m| <= rkcut) and adds the mode's energy and
-// virial terms, weighted for the half spectrum, to ev.  mh2 = m2/L2 and s2
-// (+1 on the k2 Nyquist plane, else -1) belong to k2; b1 b2 b3 are the
-// B-spline moduli of h, k2, k3.  ENE false: eterm only.
-template <bool ENE>
-__device__ __forceinline__ double conv_mode(const ConvArgs &ca, int h, int k3, double mh2,
-                                            double s2, double b1, double b2, double b3,
-                                            double zx, double zy, double (&ev)[8]) {
-  const int K1 = ca.K[0], K3 = ca.K[2];
-  const int nf1 = (K1 + 1) / 2, nf3 = (K3 + 1) / 2;
-  const int m1 = (h < nf1) ? h : h - K1;
-  const int m3 = (k3 < nf3) ? k3 : k3 - K3;
-  const double mh1 = ca.recip[0] * m1, mh3 = ca.recip[2] * m3;
-  // the rkcut test decides modes that lie on the sphere (e.g. integer
-  // |k|^2 = (rkcut L)^2): |m|^2 in the reference's rounding, no contraction
-  const double msq = msq_nc(mh1, mh2, mh3);
-  double eterm = 0.0;
-  if (msq <= ca.rk2) {
-    const double denom = ca.pivol * b1 * b2 * b3 * msq;
-    const double ex = exp(-ca.fac * msq);
-    eterm = ex / denom;
-    if (!ENE) return eterm;
-    const double vterm = 2.0 * (ca.fac * msq + 1.0) / msq;
-    const double struc2 = zx * zx + zy * zy;
-    const bool single = (h == 0) || ((K1 & 1) == 0 && h == K1 / 2);
-    const double w = single ? 1.0 : 2.0;
-    const double s3 = ((K3 & 1) == 0 && k3 == K3 / 2) ? 1.0 : -1.0;
-    const double w12 = single ? 1.0 : 1.0 - s2;        // s1 = -1
-    const double w13 = single ? 1.0 : 1.0 - s3;
-    const double w23 = single ? 1.0 : 1.0 + s2 * s3;
-    double wgt = eterm * struc2;
-    if (ca.ifnetq) {
-      const double e2 = ex * ca.netq / (ca.pivol * msq);
-      ev[1] += w * (e2 * (-1.0 + 2.0 * ca.fac * msq));
-      wgt = wgt - e2;
-    }
-    ev[0] += w * eterm * struc2;
-    ev[2] += w * wgt * (vterm * mh1 * mh1 - 1.0);
-    ev[3] += w * wgt * (vterm * mh2 * mh2 - 1.0);
-    ev[4] += w * wgt * (vterm * mh3 * mh3 - 1.0);
-    ev[5] += w12 * wgt * (vterm * mh1 * mh2);
-    ev[6] += w13 * wgt * (vterm * mh1 * mh3);
-    ev[7] += w23 * wgt * (vterm * mh2 * mh3);
-  }
-  return eterm;
+// Influence function of a mode (scalar_sum, fft_pme.F90:544-690): 0 outside
+// |m| <= rkcut; msq = |m|^2 as msq_nc rounds it (the rkcut test decides modes
+// that lie on the sphere, e.g. integer |k|^2 = (rkcut L)^2), b1 b2 b3 the
+// B-spline moduli.
+__device__ __forceinline__ double conv_eterm(const ConvArgs &ca, double msq, double b1, double b2,
+                                             double b3) {
+  if (!(msq <= ca.rk2)) return 0.0;
+  const double denom = ca.pivol * b1 * b2 * b3 * msq;
+  return exp(-ca.fac * msq) / denom;
 }
 
-// The same mode with exp(-fac |m|^2) taken as the product of per-axis factors
-// exp(-fac mh_d^2) and the moduli as reciprocals, so that a mode costs one
-// division.  e12 = exp(-fac (mh1^2 + mh2^2)) as a product, r12 = 1/(pi V b1 b2),
-// e3 = exp(-fac mh3^2), r3 = 1/b3; the cutoff test is the reference's.
-// ENE false: eterm only.
+// The same for mode (h, k2, k3), and its energy and virial terms, weighted for
+// the half spectrum, added to ev.  exp(-fac |m|^2) is the product of per-axis
+// factors exp(-fac mh_d^2) and the moduli are reciprocals, so that a mode costs
+// one division: e12 = exp(-fac (mh1^2 + mh2^2)) as a product, r12 = 1/(pi V b1
+// b2), e3 = exp(-fac mh3^2), r3 = 1/b3; s2 is +1 on the k2 Nyquist plane, else
+// -1.  The cutoff test is the reference's.  ENE false: eterm only.
 template <bool ENE>
 __device__ __forceinline__ double conv_mode_f(const ConvArgs &ca, int h, int k3, double mh1,
                                               double mh2, double s2, double e12, double r12,
@@ -1527,14 +1491,12 @@ __global__ __launch_bounds__(256) void k_fft_z_vir(void *cgrid, int TW, FftPlan 
     if (h >= H) continue;
     double g = 0.0;
     if (h != 0 || k2 != 0 || k3 != 0) {
-      double ev[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      const double eterm =
-          conv_mode<false>(ca, h, k3, mh2, s2, sb1[l], bsp2, sb3[k3], 0.0, 0.0, ev);
+      const int m1 = (h < nf1) ? h : h - K1;
+      const int m3 = (k3 < nf3) ? k3 : k3 - K3;
+      const double mh1 = ca.recip[0] * m1, mh3 = ca.recip[2] * m3;
+      const double msq = msq_nc(mh1, mh2, mh3);
+      const double eterm = conv_eterm(ca, msq, sb1[l], bsp2, sb3[k3]);
       if (eterm != 0.0) {
-        const int m1 = (h < nf1) ? h : h - K1;
-        const int m3 = (k3 < nf3) ? k3 : k3 - K3;
-        const double mh1 = ca.recip[0] * m1, mh3 = ca.recip[2] * m3;
-        const double msq = msq_nc(mh1, mh2, mh3);
         const double vterm = 2.0 * (ca.fac * msq + 1.0) / msq;
         const double ma = a == 0 ? mh1 : (a == 1 ? mh2 : mh3);
         const double mb = b == 0 ? mh1 : (b == 1 ? mh2 : mh3);
