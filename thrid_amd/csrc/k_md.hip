@@ -32,7 +32,7 @@ __device__ __forceinline__ double drift1(double x, double v, double dt) { return
 
 // With the Nose-Hoover chain on, the half kick is the thermostatted update
 // v exp(-dt vxi1/2) + F/m bbv (moldyn_nhc.F90:1301-1302, 1589-1590); nhc
-// points at the two factors {exp(-dt vxi1/2), bbv} that k_nhc_half keeps on
+// points at the two factors {exp(-dt vxi1/2), bbv} that the chain keeps on
 // the device, or is null (plain NVE).
 // With streaming velocities (strm), the chain scales the velocity relative to
 // the atom's streaming velocity vs and adds vs back: ((v - vs) exp(-dt
@@ -527,10 +527,11 @@ __global__ __launch_bounds__(64) void k_rattle_v(ConsArgs a) {
 // relative to the streaming velocity when vstrm is given (calkin.F90:98,
 // nhcint.F90:53-54); with skip, the atoms registered in a Langevin region
 // are left out
-__device__ __forceinline__ void ke_record(int n, const double *__restrict__ vel,
-                                          const double *__restrict__ minv, double *rec,
-                                          const int32_t *__restrict__ skip,
-                                          const double *__restrict__ vstrm) {
+__global__ __launch_bounds__(256) void k_md_ke(int n, const double *__restrict__ vel,
+                                               const double *__restrict__ minv,
+                                               double *__restrict__ rec,
+                                               const int32_t *__restrict__ skip,
+                                               const double *__restrict__ vstrm) {
   double ev[1] = {0.0};
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n && !(skip && skip[i] >= 0)) {
@@ -542,14 +543,6 @@ __device__ __forceinline__ void ke_record(int n, const double *__restrict__ vel,
   }
   block_record<1, 4>(ev, rec + (size_t)blockIdx.x * PGK_REC);
 }
-__global__ __launch_bounds__(256) void k_md_ke(int n, const double *__restrict__ vel,
-                                               const double *__restrict__ minv,
-                                               double *__restrict__ rec,
-                                               const int32_t *__restrict__ skip,
-                                               const double *__restrict__ vstrm) {
-  ke_record(n, vel, minv, rec, skip, vstrm);
-}
-
 
 // ---- Nose-Hoover chain ----------------------------------------------------
 #define PGK_NHC_MAX 10   // maxnhc (md_global.F90:58)
@@ -578,8 +571,17 @@ __device__ __forceinline__ double nhc_mid(const double (&q)[PGK_NHC_MAX],
 // sized for the longest chain and indexed with constants, so they stay in
 // registers; links past the chain hold v = 0 and are never stored.  st:
 // [3m+2] = xlogs, vlogs, qmass, exp(-dt vxi1/2), bbv.
-__device__ __forceinline__ void nhc_chain(const NhcArgs &p, int times, const double *rec,
-                                          double *st) {
+// A step whose velocities nothing reads before the next step's opening call
+// makes that call here as well (times = 2): both calls see the same records,
+// and two launches of the serial chain (8.1 us each) become one of 15.5; the
+// chain itself, one thread's exponentials, bounds it (reciprocals of the masses
+// gained nothing).  The records keep a launch of their own: integrated by their
+// last block, every block's device-wide fence made the launch grow with the
+// system (16 us at 12,000 atoms, 38 at 100,000, 256 at 900,000, against 4-7 and
+// 15.5), and a step was 1-4 us slower at every size.
+__global__ __launch_bounds__(256) void k_nhc(NhcArgs p, int times,
+                                             const double *__restrict__ rec,
+                                             double *__restrict__ st) {
 #pragma clang fp contract(off)
   double t = 0.0;
   for (int b = threadIdx.x; b < p.nrec; b += 256) t += rec[(size_t)b * PGK_REC];
@@ -637,35 +639,6 @@ __device__ __forceinline__ void nhc_chain(const NhcArgs &p, int times, const dou
   const double poly = 1.0 + a2 * (e2 + a2 * (e4 + a2 * (e6 + a2 * e8)));
   st[3 * m] = ex4 * ex4;
   st[3 * m + 1] = ex4 * poly * 0.5 * p.dt;
-}
-
-__global__ __launch_bounds__(256) void k_nhc_half(NhcArgs p, const double *__restrict__ rec,
-                                                  double *__restrict__ st) {
-  nhc_chain(p, 1, rec, st);
-}
-
-// The records and the chain in one launch: the last block to write its record
-// integrates (*done counts the blocks and is left at zero).  A step whose
-// velocities nothing reads before the next step's opening call makes that
-// call here as well (times = 2): both calls see the same records, and three
-// launches of the serial chain become one.  18,000-atom slab: 4.3 + 8.1 + 8.1
-// -> 19.0 us and two gaps less, 230.6 -> 226.4 us a step; the chain itself, one
-// thread's exponentials, bounds it (reciprocals of the masses gained nothing).
-__global__ __launch_bounds__(256) void k_md_ke_nhc(int n, const double *__restrict__ vel,
-                                                   const double *__restrict__ minv, double *rec,
-                                                   const int32_t *__restrict__ skip,
-                                                   const double *__restrict__ vstrm, NhcArgs p,
-                                                   int times, double *st, int32_t *done) {
-  __shared__ bool s_last;
-  ke_record(n, vel, minv, rec, skip, vstrm);
-  __threadfence();    // the record is visible to the device before it is counted
-  __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(done, 1) == (int)gridDim.x - 1;
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();    // and the others' records to this block
-  if (threadIdx.x == 0) *done = 0;
-  nhc_chain(p, times, rec, st);
 }
 
 ConsArgs cons_args(pgk_ctx *c) {
@@ -782,9 +755,9 @@ static NhcArgs nhc_args(pgk_ctx *c) {
   return p;
 }
 
-// one nhcint call on the kinetic-energy records already in d_md_kenhc
-int pgk_md_nhc_half(pgk_ctx *c) {
-  k_nhc_half<<<1, 256, 0, c->stream>>>(nhc_args(c), c->d_md_kenhc, c->d_md_nhc);
+// one or two nhcint calls on the kinetic-energy records already in d_md_kenhc
+int pgk_md_nhc_chain(pgk_ctx *c, int times) {
+  k_nhc<<<1, 256, 0, c->stream>>>(nhc_args(c), times, c->d_md_kenhc, c->d_md_nhc);
   HIP_CHECK(hipGetLastError());
   return PGK_OK;
 }
@@ -792,11 +765,6 @@ int pgk_md_nhc_half(pgk_ctx *c) {
 // the chain's records of the current velocities into d_md_kenhc, and one or
 // two nhcint calls on them
 int pgk_md_ke_nhc(pgk_ctx *c, int times) {
-  const int n = c->natom;
-  k_md_ke_nhc<<<pgk_grid_blocks(n, 256), 256, 0, c->stream>>>(
-      n, c->d_md_vel, c->d_md_minv, c->d_md_kenhc, c->md_lt_nreg ? c->d_lt_reg : nullptr,
-      c->md_lt_nstrm ? c->d_md_vstrm : nullptr, nhc_args(c), times, c->d_md_nhc,
-      reinterpret_cast<int32_t *>(c->d_md_nhc + 3 * c->md_nhc_m + 2));
-  HIP_CHECK(hipGetLastError());
-  return PGK_OK;
+  const int rc = pgk_md_ke(c, c->d_md_kenhc, true);
+  return rc ? rc : pgk_md_nhc_chain(c, times);
 }

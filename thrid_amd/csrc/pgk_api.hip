@@ -1729,7 +1729,7 @@ struct MdRunner {
       opened = false;
       return PGK_OK;
     }
-    return c->md_lt_nreg ? pgk_md_ke_nhc(c, 1) : pgk_md_nhc_half(c);
+    return c->md_lt_nreg ? pgk_md_ke_nhc(c, 1) : pgk_md_nhc_chain(c, 1);
   }
   // A step that samples nothing is followed by another of this run (the last
   // one samples), so its closing launch makes that step's opening call as
@@ -2035,7 +2035,7 @@ int pgk_md_nhc(pgk_ctx *c, const pgk_nhc_desc *nhc) {
   }
   // kT in eref, masses in eref fs^2 (prepmd.F90:515-518)
   const double gkt = 1.380649e-23 / 6.9511042e-21 * nhc->temperature;
-  std::vector<double> st((size_t)3 * m + 3, 0.0);
+  std::vector<double> st((size_t)3 * m + 2, 0.0);
   for (int i = 0; i < m; i++) {
     st[i] = nhc->xlogs ? nhc->xlogs[i] : 0.0;
     st[m + i] = nhc->vlogs ? nhc->vlogs[i] : 0.0;

@@ -318,7 +318,7 @@ struct pgk_ctx {
   int md_nhc_m = 0, md_nhc_nyosh = 1, md_nhc_next = 1;
   double md_nhc_gkt = 0.0, md_nhc_gnkt = 0.0;
   double md_nhc_ys[5] = {};
-  double *d_md_nhc = nullptr;      // [3m+3]: xlogs, vlogs, qmass, exp(-dt vxi1/2), bbv, block count
+  double *d_md_nhc = nullptr;      // [3m+2]: xlogs, vlogs, qmass, exp(-dt vxi1/2), bbv
   // region Langevin thermostat (pgk_md_langevin); off when md_lt_nreg == 0.
   // Registration units: a molecule by its centre of mass (ucom 1) or one
   // atom (ucom 0), CSR ustart over uatom.
@@ -422,7 +422,7 @@ int pgk_md_kick_drift(pgk_ctx *c, const double *f, double dt, const double *fl, 
 int pgk_md_kick(pgk_ctx *c, const double *f, double dt, const double *fl, double dtl);
 int pgk_md_rattle_v(pgk_ctx *c);
 int pgk_md_ke(pgk_ctx *c, double *rec, bool nhc = false);
-int pgk_md_nhc_half(pgk_ctx *c);
+int pgk_md_nhc_chain(pgk_ctx *c, int times);
 int pgk_md_ke_nhc(pgk_ctx *c, int times);
 int pgk_md_lt_register(pgk_ctx *c);      // assign atoms to the Langevin regions
 int pgk_md_strm_assign(pgk_ctx *c);      // streaming velocities at the current positions
