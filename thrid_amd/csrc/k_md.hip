@@ -573,12 +573,12 @@ __device__ __forceinline__ double nhc_mid(const double (&q)[PGK_NHC_MAX],
 // [3m+2] = xlogs, vlogs, qmass, exp(-dt vxi1/2), bbv.
 // A step whose velocities nothing reads before the next step's opening call
 // makes that call here as well (times = 2): both calls see the same records,
-// and two launches of the serial chain (8.1 us each) become one of 15.5; the
+// and two launches of the serial chain (8.1 us each) become one of 12.7; the
 // chain itself, one thread's exponentials, bounds it (reciprocals of the masses
 // gained nothing).  The records keep a launch of their own: integrated by their
 // last block, every block's device-wide fence made the launch grow with the
 // system (16 us at 12,000 atoms, 38 at 100,000, 256 at 900,000, against 4-7 and
-// 15.5), and a step was 1-4 us slower at every size.
+// 13-16), and a step was 1-4 us slower at every size.
 __global__ __launch_bounds__(256) void k_nhc(NhcArgs p, int times,
                                              const double *__restrict__ rec,
                                              double *__restrict__ st) {
