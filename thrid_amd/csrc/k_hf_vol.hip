@@ -334,9 +334,10 @@ __global__ __launch_bounds__(256) void k_hf_pairs_vol(HfVolArgs p, HfDev h,
             const R t2 = rinv2 * (R)lj[2 * tp + 1];
             const R t6 = t2 * t2 * t2;
             const R t12 = t6 * t6;
-            // (0 x infinity at a contact of atoms without LJ is nothing)
-            ev = ep != R(0) ? ep * (t12 - (R)2 * t6) : R(0);
-            fv = ep != R(0) ? (R)12 * ep * (t12 - t6) * rinv2 : R(0);
+            if (ep != R(0)) {   // (0 x infinity at a contact of atoms without LJ is nothing)
+              ev = ep * (t12 - (R)2 * t6);
+              fv = (R)12 * ep * (t12 - t6) * rinv2;
+            }
           }
           double sc = seg ? (double)fc * rw : 0.0, sv = seg ? (double)fv * rw : 0.0;
           const bool whole = h.reversed || !(fabs(sc) < kVolMax && fabs(sv) < kVolMax);
